@@ -9,6 +9,10 @@
 // ((v00*(1-ly))*(1-lx)) + ((v01*(1-ly))*lx) + ((v10*ly)*(1-lx)) + ((v11*ly)*lx).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
+#include "dcn_device.hpp"
 #include "dcn_internal.hpp"
 
 #pragma clang fp contract(off)
@@ -124,238 +128,383 @@ hipError_t launch_direct(const KShape& s, const T* in, const T* off, const T* ma
     return hipGetLastError();
 }
 
-// ---- FP32 with shared samples ----------------------------------------------------------
+// ---- shared samples --------------------------------------------------------------------
 // direct_kernel evaluates every bilinear sample once per output channel. Here a workgroup
-// owns 16 output pixels x 64 output channels: each (pixel, ic, tap) sample is evaluated
-// once, as sampled * mask, into LDS, and every output channel of the workgroup reads it
-// there. Each output still sums bias, then ic, ky, kx in order, as
+// owns 16 output pixels x OC output channels of one group: each (pixel, ic, tap) sample is
+// evaluated once, as sampled * mask, into LDS, and every output channel of the workgroup
+// reads it there. Each output still sums bias, then ic, ky, kx in order, as
 // sum + ((sampled * mask) * weight) with one rounding per operation (no contraction), so
-// the result is direct_kernel's, and the oracle's, bit for bit. groups == 1 only.
+// the result is direct_kernel's, and the oracle's, bit for bit.
 //
-// Lanes: pixel p = tid % 16, output-channel group q = tid / 16 of OCL channels (OCL
-// independent chains per lane; 64 / OCL * 16 threads). The input channels go by in stages of 8
-// (J = 8 * KA samples per pixel): stage c + 1's offsets, masks and weights are loaded
-// before stage c's chains, its corner gathers issued halfway through them and its
-// samples finished after them, so the loads' latency hides behind the chains.
+// Bound: one FP32 multiply and one add per (output, ic, tap), 604 M lane operations at
+// 1x128x64x64 -> 64, 15.4 us at 64 per CU and clock. With both operands read from LDS a wave's
+// two 16-byte reads per 4 taps cost 64 of a CU's LDS clocks for 32 of its VALU's (34.9 us),
+// so only the samples come from LDS: lane l holds pixel l % 16 of output channels
+// OCL * (l / 16) + e, the 16 lanes of a row share their channels, and each keeps one weight of
+// every 16 consecutive (ic, tap) in a register that the multiply reads through a DPP row
+// broadcast (4.2 clocks against 3.1 for a plain multiply, measured). Weights go from memory
+// to registers, one stage ahead. 34.9 -> 28.0 us FP32; FP16 2x128x45x61 -> 64, which ran
+// direct_kernel, 1584 -> 48.7 us (343 workgroups on 256 CUs; 45x61 alone 25.5 us). The corner
+// gathers come next: a pixel's samples are a cache line per channel and corner row, so the
+// two columns of a row are one load (four single loads: 38.6 us against 28.0).
+//
+// NW waves run the chains and SW more sample: the input channels go by in stages of 16
+// (J = 16 * KA samples per pixel, KA chunks of 16); while the chains consume stage st from
+// one LDS buffer, the sampling waves fill the other with stage st + 1 and request the
+// offsets of stage st + 2. In the chains' own waves each wait for a weight would
+// also wait for the gathers. A sampling item is one (pixel, tap) of CPI channels that
+// share an offset group: position and corner weights once, CPI x 4 corner loads.
 constexpr int kSharedPix = 16;
-constexpr int kSharedOc = 64;
-constexpr int kSharedCh = 8;
+constexpr int kSharedCh = 16;
 
-template <int KA, int OCL>
-struct SharedLayout {
-    static constexpr int NT = kSharedPix * kSharedOc / OCL;      // threads
-    static constexpr int J = kSharedCh * KA;  // samples per pixel and stage
-    static constexpr int JP = J + 4;          // padded row (floats), rows stay 16-byte aligned
-    static constexpr int PER = (kSharedPix * J + NT - 1) / NT;       // samples per thread
-    static constexpr int WPER = (kSharedOc * J / 4 + NT - 1) / NT;   // weight float4s per thread
+template <typename T>
+struct SharedArgs {
+    const T *input, *offset, *mask, *weight, *bias;
+    T* output;
+    KShape s;
+    long pixels;
+    int cpg, opg, cpog;   // channels per group, output channels per group, channels per offset group
+    int oc_tiles;         // workgroups along one group's output channels
+    uint32_t off_bytes, mask_bytes, weight_bytes;
 };
 
-template <int KA, int OCL>
-__global__ __launch_bounds__((SharedLayout<KA, OCL>::NT)) void direct_shared_f32_kernel(
-    const float* __restrict__ input, const float* __restrict__ offset, const float* __restrict__ mask,
-    const float* __restrict__ weight, const float* __restrict__ bias, float* __restrict__ output, KShape s,
-    long pixels) {
-    using L = SharedLayout<KA, OCL>;
-    constexpr int J = L::J, JP = L::JP, NT = L::NT;
-    __shared__ __attribute__((aligned(16))) float sm[2][kSharedPix][JP];  // sampled * mask
-    __shared__ __attribute__((aligned(16))) float wn[2][kSharedOc][JP];   // weights [oc][j]
-    const int tid = threadIdx.x;
-    const int oc_base = blockIdx.y * kSharedOc;
-    const long pix0 = (long)blockIdx.x * kSharedPix;
+template <int KA, int CPI>
+struct SharedLayout {
+    static constexpr int J = kSharedCh * KA;
+    static constexpr int JP = J + 4;  // padded row (floats): 16-byte aligned rows, odd in 16-byte units
+    static constexpr int ITEMS = kSharedPix * KA * (kSharedCh / CPI);
+    static constexpr int SW = ITEMS >= 512 ? 8 : (ITEMS + 63) / 64;  // sampling waves
+    static constexpr int PER = (ITEMS + 64 * SW - 1) / (64 * SW);    // items per sampling lane
+};
 
-    // The pixel this thread samples (every sample of a thread has pixel tid % 16).
-    const int sp = tid & 15;
-    const long spix = min(pix0 + sp, pixels - 1);
-    const long plane = (long)s.Ho * s.Wo;
-    const long sn = spix / plane;
-    const long sspatial = spix - sn * plane;
-    const int soy = (int)(sspatial / s.Wo);
-    const int sox = (int)(sspatial - (long)soy * s.Wo);
-    const long off_base = sn * 2 * s.og * KA * plane + sspatial;
-    const long mask_base = sn * s.og * KA * plane + sspatial;
-    const long in_plane = (long)s.H * s.W;
-    const int cpog = s.Cin / s.og;
-    const int KW = s.KW;
-    const long wrow = (long)s.Cin * KA;  // weights per output channel (groups == 1)
-
-    float ofy[L::PER], ofx[L::PER], mk[L::PER];
-    float4 wreg[L::WPER];
-    long ibase[L::PER];
-    float v[L::PER][4], ly[L::PER], lx[L::PER];
-
-    auto sample_jj = [&](int i) { return (tid >> 4) + NT / 16 * i; };
-    // Stage st's offsets, masks and weights into registers.
-    auto load_stage = [&](int st) {
-        const int ic0 = st * kSharedCh;
-#pragma unroll
-        for (int i = 0; i < L::PER; ++i) {
-            const int jj = sample_jj(i);
-            if (jj >= J) continue;
-            const int ic = ic0 + jj / KA;
-            const int k = jj % KA;
-            const int og = ic / cpog;
-            const long oc_ch = 2L * (og * KA + k);
-            ofy[i] = offset[off_base + oc_ch * plane];
-            ofx[i] = offset[off_base + (oc_ch + 1) * plane];
-            mk[i] = mask[mask_base + (long)(og * KA + k) * plane];
-            ibase[i] = (sn * s.Cin + ic) * in_plane;
-        }
-#pragma unroll
-        for (int i = 0; i < L::WPER; ++i) {
-            const int t = tid + NT * i;
-            const int oc_l = t / (J / 4);
-            const int j4 = t - oc_l * (J / 4);
-            wreg[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (oc_l < kSharedOc && oc_base + oc_l < s.Cout)
-                wreg[i] = *reinterpret_cast<const float4*>(weight + (long)(oc_base + oc_l) * wrow +
-                                                           (long)ic0 * KA + 4 * j4);
-        }
-    };
-    // Coordinates and the four corner loads (a corner outside the input reads 0).
-    auto gather_stage = [&]() {
-#pragma unroll
-        for (int i = 0; i < L::PER; ++i) {
-            const int jj = sample_jj(i);
-            if (jj >= J) continue;
-            const int k = jj % KA;
-            const int ky = k / KW;
-            const int kx = k - ky * KW;
-            const float y = (float)(soy * s.sh - s.ph + ky * s.dh) + ofy[i];
-            const float x = (float)(sox * s.sw - s.pw + kx * s.dw) + ofx[i];
-            const float fy = floorf(y), fx = floorf(x);
-            ly[i] = y - fy;
-            lx[i] = x - fx;
-            // floor() of a finite float converts exactly once clamped (clamped values are
-            // out of bounds either way; NaN clamps to the lower bound).
-            const int y0 = (int)fminf(fmaxf(fy, -4.0f), (float)s.H + 4.0f);
-            const int x0 = (int)fminf(fmaxf(fx, -4.0f), (float)s.W + 4.0f);
-            const bool ry0 = y0 >= 0 && y0 < s.H, ry1 = y0 + 1 >= 0 && y0 + 1 < s.H;
-            const bool rx0 = x0 >= 0 && x0 < s.W, rx1 = x0 + 1 >= 0 && x0 + 1 < s.W;
-            const long b = ibase[i] + (long)y0 * s.W + x0;
-            v[i][0] = (ry0 && rx0) ? input[b] : 0.0f;
-            v[i][1] = (ry0 && rx1) ? input[b + 1] : 0.0f;
-            v[i][2] = (ry1 && rx0) ? input[b + s.W] : 0.0f;
-            v[i][3] = (ry1 && rx1) ? input[b + s.W + 1] : 0.0f;
-        }
-    };
-    // The samples (DeformConvCPU.bilinear's association) times the mask, and the
-    // weights, into LDS buffer nb.
-    auto store_stage = [&](int nb) {
-#pragma unroll
-        for (int i = 0; i < L::PER; ++i) {
-            const int jj = sample_jj(i);
-            if (jj >= J) continue;
-            const float a = 1.0f - ly[i], c = 1.0f - lx[i];
-            const float sampled = v[i][0] * a * c + v[i][1] * a * lx[i] + v[i][2] * ly[i] * c +
-                                  v[i][3] * ly[i] * lx[i];
-            sm[nb][sp][jj] = sampled * mk[i];
-        }
-#pragma unroll
-        for (int i = 0; i < L::WPER; ++i) {
-            const int t = tid + NT * i;
-            const int oc_l = t / (J / 4);
-            const int j4 = t - oc_l * (J / 4);
-            if (oc_l < kSharedOc) *reinterpret_cast<float4*>(&wn[nb][oc_l][4 * j4]) = wreg[i];
-        }
-    };
-
-    const int p = tid & 15;
-    const int q = tid >> 4;
-    float acc[OCL];
-#pragma unroll
-    for (int e = 0; e < OCL; ++e) acc[e] = oc_base + OCL * q + e < s.Cout ? bias[oc_base + OCL * q + e] : 0.0f;
-    // sum + (sm * w) for samples [4 * lo, 4 * hi) of buffer nb, in order.
-    auto chain = [&](int nb, int lo, int hi) {
-#pragma unroll 3
-        for (int j4 = lo; j4 < hi; ++j4) {
-            const float4 sv = *reinterpret_cast<const float4*>(&sm[nb][p][4 * j4]);
-            float4 w4[OCL];
-#pragma unroll
-            for (int e = 0; e < OCL; ++e) w4[e] = *reinterpret_cast<const float4*>(&wn[nb][OCL * q + e][4 * j4]);
-#pragma unroll
-            for (int e = 0; e < OCL; ++e) acc[e] = acc[e] + sv.x * w4[e].x;
-#pragma unroll
-            for (int e = 0; e < OCL; ++e) acc[e] = acc[e] + sv.y * w4[e].y;
-#pragma unroll
-            for (int e = 0; e < OCL; ++e) acc[e] = acc[e] + sv.z * w4[e].z;
-#pragma unroll
-            for (int e = 0; e < OCL; ++e) acc[e] = acc[e] + sv.w * w4[e].w;
-        }
-    };
-
-    const int stages = s.Cin / kSharedCh;
-    load_stage(0);
-    gather_stage();
-    store_stage(0);
-    __syncthreads();
-    for (int st = 0; st < stages; ++st) {
-        const int nb = st & 1;
-        const bool more = st + 1 < stages;
-        if (more) load_stage(st + 1);
-        chain(nb, 0, J / 8);
-        if (more) gather_stage();
-        chain(nb, J / 8, J / 4);
-        if (more) store_stage(nb ^ 1);
-        __syncthreads();
-    }
-
-    const long pix = pix0 + p;
-    if (pix >= pixels) return;
-    const long n = pix / plane;
-    const long spatial = pix - n * plane;
-#pragma unroll
-    for (int e = 0; e < OCL; ++e) {
-        const int oc = oc_base + OCL * q + e;
-        if (oc < s.Cout) output[(n * s.Cout + oc) * plane + spatial] = acc[e];
-    }
+template <typename T>
+__device__ __forceinline__ float load_widened(__amdgpu_buffer_rsrc_t r, uint32_t element, uint32_t soff = 0) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(element * 4u), (int)soff, 0));
+    return dev::load_half(r, element * 2u, soff);
 }
 
-template <int KA>
-hipError_t launch_shared_f32(const KShape& s, const float* in, const float* off, const float* mask,
-                             const float* w, const float* b, float* out, hipStream_t stream) {
-    // One channel per lane (1024 threads, 4 waves per SIMD) measured 38.8 us at C1
-    // against 48.4 us with two and 63.3 us with four: the chains are latency-bound and
-    // the extra waves hide the LDS and gather latency better than the extra ILP does.
-    constexpr int OCL = 1;
-    const long pixels = (long)s.B * s.Ho * s.Wo;
-    const dim3 grid((unsigned)((pixels + kSharedPix - 1) / kSharedPix),
-                    (unsigned)((s.Cout + kSharedOc - 1) / kSharedOc));
-    hipLaunchKernelGGL((direct_shared_f32_kernel<KA, OCL>), grid, dim3(SharedLayout<KA, OCL>::NT), 0, stream, in,
-                       off, mask, w, b, out, s, pixels);
+// Two neighbouring elements of a row, one load (any element alignment).
+template <typename T>
+struct Pair;
+template <>
+struct Pair<float> {
+    float2 v;
+};
+template <>
+struct Pair<uint16_t> {
+    uint32_t v;
+};
+template <typename T>
+__device__ __forceinline__ Pair<T> load_pair(const T* p) {
+    Pair<T> r;
+    __builtin_memcpy(&r.v, p, 2 * sizeof(T));
+    return r;
+}
+__device__ __forceinline__ float first(const Pair<float>& p) { return p.v.x; }
+__device__ __forceinline__ float second(const Pair<float>& p) { return p.v.y; }
+__device__ __forceinline__ float first(const Pair<uint16_t>& p) { return widen((uint16_t)p.v); }
+__device__ __forceinline__ float second(const Pair<uint16_t>& p) { return widen((uint16_t)(p.v >> 16)); }
+
+// t[i] = s[i] * w of lane 4 Q + i of the caller's row of 16 lanes. In assembly because the
+// compiler makes the broadcasts of a whole stage first, as moves, and spills them. A DPP
+// operand may not have been written by the two vector instructions before: s_nop at the
+// chunk's first use of w, which the volatile order keeps first.
+template <int Q>
+__device__ __forceinline__ void row_products(const float4& s, float w, float (&t)[4]) {
+    if constexpr (Q == 0)
+        __asm__ volatile(
+            "s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %4, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %2, %4, %7 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %3, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf"
+            : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])
+            : "v"(w), "v"(s.x), "v"(s.y), "v"(s.z), "v"(s.w), "n"(4 * Q), "n"(4 * Q + 1), "n"(4 * Q + 2), "n"(4 * Q + 3));
+    else
+        __asm__ volatile(
+            "v_mul_f32_dpp %0, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %4, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %2, %4, %7 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %3, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf"
+            : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])
+            : "v"(w), "v"(s.x), "v"(s.y), "v"(s.z), "v"(s.w), "n"(4 * Q), "n"(4 * Q + 1), "n"(4 * Q + 2), "n"(4 * Q + 3));
+}
+
+// The first `count` of samples 4 Q .. 4 Q + 3 of a chunk: sum + (sample * weight), in order.
+template <int Q, int OCL, bool ALL>
+__device__ __forceinline__ void chain4(float (&acc)[OCL], const float4& s, const float (&w)[OCL], int count) {
+    float t[OCL][4];
+#pragma unroll
+    for (int e = 0; e < OCL; ++e) row_products<Q>(s, w[e], t[e]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < OCL; ++e)
+            if (ALL || i < count) acc[e] = acc[e] + t[e][i];
+}
+
+template <typename T, int KA, int NW, int OCL, int CPI>
+__global__ __launch_bounds__(64 * (NW + SharedLayout<KA, CPI>::SW)) void shared_kernel(SharedArgs<T> a) {
+    using L = SharedLayout<KA, CPI>;
+    constexpr int JP = L::JP;
+    __shared__ __attribute__((aligned(16))) float sm[2][kSharedPix][JP];  // sampled * mask
+    const KShape& s = a.s;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p = threadIdx.x & 15;
+    const int group = blockIdx.y / a.oc_tiles;
+    const long pix0 = (long)blockIdx.x * kSharedPix;
+    const long plane = (long)s.Ho * s.Wo;
+    const long pix = min(pix0 + p, a.pixels - 1);
+    const int n = (int)(pix / plane);
+    const int spatial = (int)(pix - n * plane);
+    const int stages = (a.cpg + kSharedCh - 1) / kSharedCh;
+
+    if (wave >= NW) {
+        // Sampling waves: item t = (tap, channel block) * 16 + pixel. Lanes past the last
+        // item repeat it (the same value to the same place).
+        const int oy = spatial / s.Wo;
+        const int ox = spatial - oy * s.Wo;
+        const uint32_t in_plane = (uint32_t)s.H * s.W;
+        const __amdgpu_buffer_rsrc_t offr = dev::make_rsrc(a.offset, a.off_bytes);
+        const __amdgpu_buffer_rsrc_t maskr = dev::make_rsrc(a.mask, a.mask_bytes);
+        int k[L::PER], ch[L::PER];
+        float y0f[L::PER], x0f[L::PER];
+#pragma unroll
+        for (int i = 0; i < L::PER; ++i) {
+            const int rest = min((int)(threadIdx.x - 64 * NW + 64 * L::SW * i) >> 4, L::ITEMS / 16 - 1);
+            k[i] = rest % KA;
+            ch[i] = rest / KA * CPI;
+            const int ky = k[i] / s.KW;
+            y0f[i] = (float)(oy * s.sh - s.ph + ky * s.dh);
+            x0f[i] = (float)(ox * s.sw - s.pw + (k[i] - ky * s.KW) * s.dw);
+        }
+        float ofy[L::PER], ofx[L::PER], mk[L::PER];
+        // Offsets and masks of stage st; channels past the group's repeat its last block.
+        auto channel = [&](int st, int i) { return min(st * kSharedCh + ch[i], a.cpg - CPI); };
+        auto load_stage = [&](int st) {
+#pragma unroll
+            for (int i = 0; i < L::PER; ++i) {
+                const int og = (group * a.cpg + channel(st, i)) / a.cpog;
+                const uint32_t m = (uint32_t)((n * s.og + og) * KA + k[i]) * (uint32_t)plane + spatial;
+                const uint32_t o = m * 2 - spatial;
+                ofy[i] = load_widened<T>(offr, o);
+                ofx[i] = load_widened<T>(offr, o + (uint32_t)plane);
+                mk[i] = load_widened<T>(maskr, m);
+            }
+        };
+        // Stage st's samples (DeformConvCPU.bilinear's association; a corner outside the
+        // input reads 0) times the mask into buffer st % 2; the next stage's offsets are
+        // requested behind the corners.
+        auto sample_stage = [&](int st, bool more) {
+            Pair<T> top[L::PER][CPI], low[L::PER][CPI];
+            float ly[L::PER], lx[L::PER], m[L::PER];
+            bool ry0[L::PER], ry1[L::PER], rx0[L::PER], rx1[L::PER], shift[L::PER];
+#pragma unroll
+            for (int i = 0; i < L::PER; ++i) {
+                const float y = y0f[i] + ofy[i];
+                const float x = x0f[i] + ofx[i];
+                m[i] = mk[i];
+                const float fy = floorf(y), fx = floorf(x);
+                ly[i] = y - fy;
+                lx[i] = x - fx;
+                // floor() of a finite float converts exactly once clamped (clamped values are
+                // out of bounds either way; NaN clamps to the lower bound).
+                const int y0 = (int)fminf(fmaxf(fy, -4.0f), (float)s.H + 4.0f);
+                const int x0 = (int)fminf(fmaxf(fx, -4.0f), (float)s.W + 4.0f);
+                ry0[i] = y0 >= 0 && y0 < s.H;
+                ry1[i] = y0 + 1 >= 0 && y0 + 1 < s.H;
+                rx0[i] = x0 >= 0 && x0 < s.W;
+                rx1[i] = x0 + 1 >= 0 && x0 + 1 < s.W;
+                // The pair of columns loaded: x0 and x0 + 1, moved into the row at its ends.
+                const int xb = min(max(x0, 0), s.W - 2);
+                shift[i] = xb != x0;
+                const uint32_t plane0 = (uint32_t)(n * s.Cin + group * a.cpg + channel(st, i)) * in_plane + xb;
+                const T* r0 = a.input + (plane0 + (uint32_t)(min(max(y0, 0), s.H - 1) * s.W));
+                const T* r1 = a.input + (plane0 + (uint32_t)(min(max(y0 + 1, 0), s.H - 1) * s.W));
+#pragma unroll
+                for (int c = 0; c < CPI; ++c) {
+                    top[i][c] = load_pair<T>(r0 + (size_t)c * in_plane);
+                    low[i][c] = load_pair<T>(r1 + (size_t)c * in_plane);
+                }
+            }
+            if (more) load_stage(st + 1);
+#pragma unroll
+            for (int i = 0; i < L::PER; ++i) {
+                const float cy = 1.0f - ly[i], cx = 1.0f - lx[i];
+                // A moved pair holds column x0 second (x0 the last column) or x0 + 1 first.
+                const bool a0 = ry0[i] && rx0[i], a1 = ry0[i] && rx1[i], b0 = ry1[i] && rx0[i], b1 = ry1[i] && rx1[i];
+#pragma unroll
+                for (int c = 0; c < CPI; ++c) {
+                    const float t0 = first(top[i][c]), t1 = second(top[i][c]);
+                    const float u0 = first(low[i][c]), u1 = second(low[i][c]);
+                    const float v00 = a0 ? (shift[i] ? t1 : t0) : 0.0f;
+                    const float v01 = a1 ? (shift[i] ? t0 : t1) : 0.0f;
+                    const float v10 = b0 ? (shift[i] ? u1 : u0) : 0.0f;
+                    const float v11 = b1 ? (shift[i] ? u0 : u1) : 0.0f;
+                    const float sampled = v00 * cy * cx + v01 * cy * lx[i] + v10 * ly[i] * cx + v11 * ly[i] * lx[i];
+                    sm[st & 1][p][(ch[i] + c) * KA + k[i]] = sampled * m[i];
+                }
+            }
+        };
+        load_stage(0);
+        for (int st = 0; st < stages; ++st) {
+            sample_stage(st, st + 1 < stages);
+            __syncthreads();  // stage st is ready; stage st - 1's buffer is free
+        }
+        if (a.cpg % kSharedCh == 0) __syncthreads();  // the chains' barrier after their last whole stage
+        return;
+    }
+
+    // Chain waves. This row's weights: chunk c of a stage is lane p's element 16 c + p of the
+    // stage's (ic, tap) run. Channels past the group's load its last one, elements past a
+    // channel's run the next one's or zero: nothing uses them.
+    const int oc0 = (blockIdx.y - group * a.oc_tiles) * (4 * NW * OCL) + (threadIdx.x >> 4) * OCL;  // in the group
+    const __amdgpu_buffer_rsrc_t wr = dev::make_rsrc(a.weight, a.weight_bytes);
+    uint32_t wbase[OCL];
+    float acc[OCL], w[KA][OCL];
+#pragma unroll
+    for (int e = 0; e < OCL; ++e) {
+        const int oc = group * a.opg + min(oc0 + e, a.opg - 1);
+        wbase[e] = (uint32_t)oc * (uint32_t)(a.cpg * KA) + p;
+        acc[e] = widen(a.bias[oc]);
+    }
+    auto load_run = [&](int j0, float (&v)[OCL]) {
+#pragma unroll
+        for (int e = 0; e < OCL; ++e) v[e] = load_widened<T>(wr, wbase[e], (uint32_t)j0 * (uint32_t)sizeof(T));
+    };
+    auto load_weights = [&](int st, int c) { load_run(st * L::J + 16 * c, w[c]); };
+    auto row4 = [&](int nb, int j) { return *reinterpret_cast<const float4*>(&sm[nb][p][j]); };
+#pragma unroll
+    for (int c = 0; c < KA; ++c) load_weights(0, c);
+    __syncthreads();
+    const int full = a.cpg / kSharedCh;  // whole stages
+#pragma unroll 1
+    for (int st = 0; st < full; ++st) {
+        const int nb = st & 1;
+#pragma unroll
+        for (int c = 0; c < KA; ++c) {
+            const float4 s0 = row4(nb, 16 * c), s1 = row4(nb, 16 * c + 4);
+            const float4 s2 = row4(nb, 16 * c + 8), s3 = row4(nb, 16 * c + 12);
+            chain4<0, OCL, true>(acc, s0, w[c], 4);
+            chain4<1, OCL, true>(acc, s1, w[c], 4);
+            chain4<2, OCL, true>(acc, s2, w[c], 4);
+            chain4<3, OCL, true>(acc, s3, w[c], 4);
+            load_weights(st + 1, c);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+    }
+    if (full < stages) {
+        // The last, partial stage: its weights again, a chunk ahead.
+        const int nb = full & 1;
+        const int count = (a.cpg - full * kSharedCh) * KA;
+        load_weights(full, 0);
+#pragma unroll 1
+        for (int c = 0; 16 * c < count; ++c) {
+            float wt[OCL];
+#pragma unroll
+            for (int e = 0; e < OCL; ++e) wt[e] = w[0][e];
+            load_run(full * L::J + 16 * (c + 1), w[0]);
+            const int left = count - 16 * c;
+            const float4 s0 = row4(nb, 16 * c), s1 = row4(nb, 16 * c + 4);
+            const float4 s2 = row4(nb, 16 * c + 8), s3 = row4(nb, 16 * c + 12);
+            if (left >= 16) {
+                chain4<0, OCL, true>(acc, s0, wt, 4);
+                chain4<1, OCL, true>(acc, s1, wt, 4);
+                chain4<2, OCL, true>(acc, s2, wt, 4);
+                chain4<3, OCL, true>(acc, s3, wt, 4);
+            } else {
+                chain4<0, OCL, false>(acc, s0, wt, left);
+                chain4<1, OCL, false>(acc, s1, wt, left - 4);
+                chain4<2, OCL, false>(acc, s2, wt, left - 8);
+                chain4<3, OCL, false>(acc, s3, wt, left - 12);
+            }
+        }
+    }
+
+    if (pix0 + p >= a.pixels) return;
+#pragma unroll
+    for (int e = 0; e < OCL; ++e)
+        if (oc0 + e < a.opg)
+            store_out(a.output, ((long)n * s.Cout + group * a.opg + oc0 + e) * plane + spatial, acc[e]);
+}
+
+template <typename T, int KA, int NW, int OCL, int CPI>
+hipError_t launch_shared_as(SharedArgs<T> a, hipStream_t stream) {
+    constexpr int OC = 4 * NW * OCL;
+    a.oc_tiles = (a.opg + OC - 1) / OC;
+    const dim3 grid((unsigned)((a.pixels + kSharedPix - 1) / kSharedPix), (unsigned)(a.s.groups * a.oc_tiles));
+    hipLaunchKernelGGL((shared_kernel<T, KA, NW, OCL, CPI>), grid, dim3(64 * (NW + SharedLayout<KA, CPI>::SW)), 0,
+                       stream, a);
     return hipGetLastError();
+}
+
+// Output channels per workgroup: the fewest whose workgroups still fit the 256 CUs at once
+// (more CUs busy beat the samples evaluated again per channel tile), else as many as the
+// group has, up to 64. Measured for 128 -> 64 channels FP32, us at 16 / 32 / 64 channels:
+// 32x32 pixels (64 pixel tiles) 17.0 / 18.4 / 22.6, 45x61 (172) 41.9 / 34.9 / 25.5, 64x64 (256)
+// 69.5 / 34.3 / 28.0. Up to 16 channels on more than 256 workgroups take two chain waves of
+// two channels per lane: 2x60x60, 4 groups of 24 -> 10, 30.3 -> 26.5 us.
+template <typename T, int KA, int CPI>
+hipError_t launch_shared_ka(const SharedArgs<T>& a, hipStream_t stream) {
+    const long tiles = (a.pixels + kSharedPix - 1) / kSharedPix * a.s.groups;
+    const auto fits = [&](int oc) { return tiles * ((a.opg + oc - 1) / oc) <= 256; };
+    if (fits(16)) return launch_shared_as<T, KA, 4, 1, CPI>(a, stream);
+    if (a.opg <= 16) return launch_shared_as<T, KA, 2, 2, CPI>(a, stream);
+    if (a.opg <= 32 || fits(32)) return launch_shared_as<T, KA, 4, 2, CPI>(a, stream);
+    return launch_shared_as<T, KA, 8, 2, CPI>(a, stream);
+}
+
+template <typename T>
+hipError_t launch_forward(const KShape& s, const T* in, const T* off, const T* mask, const T* w, const T* b, T* out,
+                          hipStream_t stream) {
+    SharedArgs<T> a{in, off, mask, w, b, out, s, (long)s.B * s.Ho * s.Wo, s.Cin / s.groups, s.Cout / s.groups,
+                    s.Cin / s.og, 0, 0, 0, 0};
+    const int ka = s.KH * s.KW;
+    // The shared kernel addresses each tensor with 32-bit byte offsets below 2^31 and its
+    // sampling positions with 32-bit integers; grid y is one workgroup column per group
+    // and channel tile.
+    const double limit = 2147483648.0;
+    const double in_bytes = (double)s.B * s.Cin * s.H * s.W * sizeof(T);
+    const double mask_bytes = (double)a.pixels * s.og * ka * sizeof(T);
+    const double weight_bytes = (double)s.Cout * a.cpg * ka * sizeof(T);
+    const double reach = std::max((double)s.Ho * s.sh + s.ph + (double)s.KH * s.dh,
+                                  (double)s.Wo * s.sw + s.pw + (double)s.KW * s.dw);
+    const bool fits = s.W >= 2 && in_bytes < limit && 2.0 * mask_bytes < limit && reach < 1e9 && s.ph > -1000000000 &&
+                      s.pw > -1000000000 && (double)s.groups * ((a.opg + 15) / 16) < 65536.0 &&
+                      weight_bytes < limit;
+    if (fits && (ka == 1 || ka == 2 || ka == 3 || ka == 4 || ka == 6 || ka == 9)) {
+        a.mask_bytes = (uint32_t)mask_bytes;
+        a.off_bytes = 2 * a.mask_bytes;
+        a.weight_bytes = (uint32_t)weight_bytes;
+        switch (ka) {
+            case 1: return launch_shared_ka<T, 1, 1>(a, stream);
+            case 2: return launch_shared_ka<T, 2, 1>(a, stream);
+            case 3: return launch_shared_ka<T, 3, 1>(a, stream);
+            case 4: return launch_shared_ka<T, 4, 1>(a, stream);
+            case 6: return launch_shared_ka<T, 6, 1>(a, stream);
+            default: break;
+        }
+        if (a.cpg % 8 == 0 && a.cpog % 8 == 0) return launch_shared_ka<T, 9, 8>(a, stream);
+        if (a.cpg % 4 == 0 && a.cpog % 4 == 0) return launch_shared_ka<T, 9, 4>(a, stream);
+        return launch_shared_ka<T, 9, 1>(a, stream);
+    }
+    return launch_direct<T>(s, in, off, mask, w, b, out, stream);
 }
 
 }  // namespace
 
-// The shared-sample kernel reads weights as float4 rows (16-byte aligned when the weight
-// pointer is and Cin % 8 == 0).
-static bool shared_f32_supported(const KShape& s, const float* w) {
-    const int ka = s.KH * s.KW;
-    return s.groups == 1 && s.Cin % kSharedCh == 0 && (uintptr_t)w % 16 == 0 &&
-           (ka == 1 || ka == 2 || ka == 3 || ka == 4 || ka == 6 || ka == 9) &&
-           (long)s.B * s.Ho * s.Wo > 0 && (long)s.B * s.Ho * s.Wo / kSharedPix < (1L << 31);
-}
-
 hipError_t launch_direct_f32(const KShape& s, const float* in, const float* off,
                              const float* mask, const float* w, const float* b, float* out,
                              hipStream_t stream) {
-    if (shared_f32_supported(s, w)) {
-        switch (s.KH * s.KW) {
-            case 1: return launch_shared_f32<1>(s, in, off, mask, w, b, out, stream);
-            case 2: return launch_shared_f32<2>(s, in, off, mask, w, b, out, stream);
-            case 3: return launch_shared_f32<3>(s, in, off, mask, w, b, out, stream);
-            case 4: return launch_shared_f32<4>(s, in, off, mask, w, b, out, stream);
-            case 6: return launch_shared_f32<6>(s, in, off, mask, w, b, out, stream);
-            default: return launch_shared_f32<9>(s, in, off, mask, w, b, out, stream);
-        }
-    }
-    return launch_direct<float>(s, in, off, mask, w, b, out, stream);
+    return launch_forward<float>(s, in, off, mask, w, b, out, stream);
 }
 
 hipError_t launch_direct_f16(const KShape& s, const uint16_t* in, const uint16_t* off,
                              const uint16_t* mask, const uint16_t* w, const uint16_t* b,
                              uint16_t* out, hipStream_t stream) {
-    return launch_direct<uint16_t>(s, in, off, mask, w, b, out, stream);
+    return launch_forward<uint16_t>(s, in, off, mask, w, b, out, stream);
 }
 
 }  // namespace dcn
