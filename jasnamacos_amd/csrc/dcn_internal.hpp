@@ -239,6 +239,18 @@ hipError_t launch_conv3x3_pair(const ConvGeometry& g1, const ConvGeometry& g2, c
                                int res1_layout, const uint16_t* res2, int res2_layout,
                                uint16_t* out, int out_layout, hipStream_t stream, int res2_coff = 0,
                                const ConvBatch& batch = ConvBatch{}, uint16_t* out2_cb8 = nullptr);
+// The same pair on larger output tiles, for many pixels (dcn_kernels_conv_wide.hip):
+// launch_conv3x3_pair runs it where conv_wide_chosen says so.
+struct ConvEnds {
+    const void *res1, *res2, *out, *out2;  // null: absent
+    int res1_layout, res2_layout, out_layout;
+};
+bool conv_wide_chosen(int height, int width, int images, const ConvEnds& ends);
+hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk1, const float* bias1,
+                                    int act1, const void* wpk2, const float* bias2, int act2, float slope,
+                                    const uint16_t* res1, int res1_layout, const uint16_t* res2, int res2_layout,
+                                    uint16_t* out, int out_layout, hipStream_t stream, int res2_coff,
+                                    const ConvBatch& batch, uint16_t* out2_cb8);
 // SPyNet (dcn_kernels_spynet.hip).
 constexpr int kSpynetMaxLevels = DCN_SPYNET_LEVELS;
 struct ConvKGeometry {

@@ -1384,6 +1384,9 @@ hipError_t launch_conv3x3_pair(const ConvGeometry& g1, const ConvGeometry& g2, c
     if (g1.cin != 64 || g1.cout != 64 || g2.cin != 64 || g2.cout != 64 || g1.h != g2.h ||
         g1.w != g2.w || g1.ksteps != kPairKsteps || g1.nbt != kConvNbc || batch.images < 1)
         return hipErrorInvalidValue;
+    if (conv_wide_chosen(g1.h, g1.w, batch.images, {res1, res2, out, out2_cb8, res1_layout, res2_layout, out_layout}))
+        return launch_conv3x3_pair_wide(g1, x_cb8, wpk1, bias1, act1, wpk2, bias2, act2, slope, res1, res1_layout,
+                                        res2, res2_layout, out, out_layout, stream, res2_coff, batch, out2_cb8);
     constexpr int NW = 8;
     PairArgs a{};
     a.xin = x_cb8;

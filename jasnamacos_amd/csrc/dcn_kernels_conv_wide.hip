@@ -1,0 +1,377 @@
+// The body's 3x3 convolutions over many pixels (large maps, batches of tiles): 16-wide
+// output tiles whose input stays in LDS, so that a weight fragment serves a hundred pixels
+// or more instead of sixteen.
+//
+// Same arithmetic, bit for bit, as dcn_kernels_conv.hip: K-step s multiplies K-blocks 4 s ..
+// 4 s + 3 (K-block tap * CB + cb) on v_mfma_f32_16x16x32_f16, the K-steps of each eighth of
+// the range [r * ksteps / 8, (r + 1) * ksteps / 8) form one accumulator chain from zero, and
+// the eight partial sums are added in order. There eight waves own an eighth each and add
+// through LDS; here one wave runs all eighths of its pixels and adds in registers. The
+// operands swap places (weights in A, pixels in B): the products and their order are the
+// same, and a lane then holds four consecutive channels of one pixel, an 8-byte store.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "dcn_device.hpp"
+#include "dcn_internal.hpp"
+
+#pragma clang fp contract(off)
+
+namespace dcn {
+namespace {
+
+using namespace dev;
+
+constexpr int kWideTW = 16;  // output tile width
+constexpr int kSteps64 = 18;  // K-steps of 64 input channels
+
+struct WidePairArgs {
+    const void* xin;
+    const void* wpk1;
+    const void* wpk2;
+    const float* bias1;
+    const float* bias2;
+    const uint16_t* res1;
+    const uint16_t* res2;
+    uint16_t* out;
+    uint16_t* out2;
+    uint32_t xin_bytes, wpk_bytes;
+    int act1, act2;
+    float slope;
+    int res1_layout, res2_layout, out_layout, res2_coff;
+    int H, W, Hp, Wp, tiles_x, tiles_image, tiles;
+    long xin_ts, res1_ts, res2_ts, out_ts, out2_ts;
+};
+
+// Four consecutive channels c .. c + 3 (c % 4 == 0) of pixel (y, x).
+struct Half4 {
+    uint32_t v[2];
+};
+__device__ __forceinline__ float half_at(const Half4& h, int i) {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)(h.v[i >> 1] >> (16 * (i & 1))));
+}
+__device__ __forceinline__ Half4 load4(const uint16_t* t, int layout, int c, int y, int x, int H, int W, int Hp, int Wp) {
+    Half4 r;
+    if (layout == kLayoutCB8) {
+        const uint2 u = *reinterpret_cast<const uint2*>(t + ((size_t)((c >> 3) * Hp + y + kPad) * Wp + x + kPad) * 8 + (c & 7));
+        r.v[0] = u.x;
+        r.v[1] = u.y;
+    } else {
+        const size_t plane = (size_t)H * W;
+        const uint16_t* p = t + (size_t)c * plane + (size_t)y * W + x;
+        const uint32_t a = p[0], b = p[plane], d = p[2 * plane], e = p[3 * plane];
+        r.v[0] = a | (b << 16);
+        r.v[1] = d | (e << 16);
+    }
+    return r;
+}
+__device__ __forceinline__ void store4(uint16_t* t, int layout, int c, int y, int x, int H, int W, int Hp, int Wp,
+                                       const Half4& h) {
+    if (layout == kLayoutCB8) {
+        *reinterpret_cast<uint2*>(t + ((size_t)((c >> 3) * Hp + y + kPad) * Wp + x + kPad) * 8 + (c & 7)) =
+            make_uint2(h.v[0], h.v[1]);
+    } else {
+        const size_t plane = (size_t)H * W;
+        uint16_t* p = t + (size_t)c * plane + (size_t)y * W + x;
+        p[0] = (uint16_t)h.v[0];
+        p[plane] = (uint16_t)(h.v[0] >> 16);
+        p[2 * plane] = (uint16_t)h.v[1];
+        p[3 * plane] = (uint16_t)(h.v[1] >> 16);
+    }
+}
+__device__ __forceinline__ Half4 pack4(const float (&f)[4]) {
+    Half4 h;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        h.v[i] = (uint32_t)__builtin_bit_cast(uint16_t, round_f16(f[2 * i])) |
+                 ((uint32_t)__builtin_bit_cast(uint16_t, round_f16(f[2 * i + 1])) << 16);
+    return h;
+}
+__device__ __forceinline__ float activate(float v, int act, float slope) {
+    if (act == 1 && v < 0.0f) v = v * slope;
+    if (act == 2 && v < 0.0f) v = 0.0f;
+    return v;
+}
+
+// 64 input channels over P 16-pixel groups and two 16-channel blocks: the sums of a tile
+// whose pixel units are in LDS as [8 blocks][PLANE], rows ROW apart, `base` the byte address
+// of each group's lane unit (block lane / 16, tap (0, 0)).
+template <int P, int PLANE, int ROW>
+__device__ __forceinline__ void gemm64(const uint8_t* lds, const uint32_t (&base)[P], __amdgpu_buffer_rsrc_t wr,
+                                       uint32_t wlane, f32x4 (&sum)[P][2]) {
+    // Everything is requested in the order it is used: the weights of the next eighth at the
+    // start of this one, the pixels of the next K-step before this one's products. Left to
+    // itself the compiler requests far more at once than the registers hold.
+    h8 B[2][3][2];
+    h8 X[2][P];
+    auto load_weights = [&](int r) {
+        __asm__ volatile("" : "+v"(wlane));
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int s = r * kSteps64 / 8 + i;
+            if (s >= (r + 1) * kSteps64 / 8) continue;
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+                B[r & 1][i][n] = __builtin_bit_cast(h8, load16(wr, wlane, (uint32_t)(s * 4 + n) * 1024u));
+        }
+    };
+    auto load_pixels = [&](int s) {
+        const int tap = s >> 1;
+        const uint32_t off = (uint32_t)((s & 1) * 4 * PLANE + tap / 3 * ROW + tap % 3) * 16u;
+#pragma unroll
+        for (int p = 0; p < P; ++p) X[s & 1][p] = *reinterpret_cast<const h8*>(lds + base[p] + off);
+    };
+    f32x4 acc[P][2];
+    load_weights(0);
+    load_pixels(0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        if (r < 7) load_weights(r + 1);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int s = r * kSteps64 / 8 + i;
+            if (s >= (r + 1) * kSteps64 / 8) continue;
+            if (s + 1 < kSteps64) load_pixels(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+                    acc[p][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(B[r & 1][i][n], X[s & 1][p],
+                                                                       i == 0 ? f32x4{} : acc[p][n], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                // A chain from +0 never ends in -0, so the first partial sum is the sum from 0.
+                if (r == 0)
+                    sum[p][n] = acc[p][n];
+                else
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sum[p][n][v] = sum[p][n][v] + acc[p][n][v];
+                __asm__ volatile("" : "+v"(sum[p][n]));  // added now: eight sets of partial sums do not fit
+            }
+    }
+}
+
+template <int TH, int PG>
+struct WidePair {
+    static constexpr int NW = 2 * PG;  // waves: PG pixel groups x 2 halves of 64 output channels
+    static constexpr int IW = kWideTW + 4, IPX = (TH + 4) * IW;     // input tile
+    static constexpr int HW = kWideTW + 2, HPX = (TH + 2) * HW;     // halo of the tile: t
+    static constexpr int P1 = ((HPX + 15) / 16 + PG - 1) / PG;  // 16-pixel groups per wave, conv1
+    static constexpr int P2 = (TH + PG - 1) / PG;          // conv2: one row each
+    static constexpr size_t lds = (size_t)8 * (IPX + HPX) * 16;
+};
+
+// Two chained 64 -> 64 convs (conv_pair_kernel's contract) on a TH x 16 output tile. The
+// input tile (two pixels more on each side) is copied into LDS once; conv1 runs over the
+// tile's halo into LDS, conv2 from there. Each wave multiplies PG-th rows of pixels by one
+// half of the output channels: a pixel fragment (LDS) serves two products and a weight
+// fragment (L1) up to P1. At 180 x 320 (240 tiles of 16 x 16, one per CU) 78 -> 17.3 us, 490
+// TFLOP/s, against conv_pair_kernel, whose 3,600 workgroups fetch all 148 KB of weights for 16
+// pixels each; 16 maps of 64 x 64 53 -> 22 us. What bounds it now: the LDS reads of the pixel
+// fragments (half a KB per product, as long as the product takes) and the latency of the two
+// dependent convs in one round of workgroups.
+template <int TH, int PG>
+__global__ __launch_bounds__((64 * WidePair<TH, PG>::NW)) void conv_pair_wide_kernel(WidePairArgs a) {
+    using L = WidePair<TH, PG>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    u32x4* xt = reinterpret_cast<u32x4*>(lds);                   // [8][IPX]
+    uint8_t* tt = lds + (size_t)8 * L::IPX * 16;                 // [8][HPX] units
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = wave >> 1;
+    const int half = wave & 1;
+    const int quarter = lane >> 4;
+
+    const int per_xcd = (a.tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= a.tiles) return;  // whole workgroup, before any barrier
+    const int z = tile / a.tiles_image;
+    const int ti = tile - z * a.tiles_image;
+    const int ty = ti / a.tiles_x;
+    const int oy0 = ty * TH;
+    const int ox0 = (ti - ty * a.tiles_x) * kWideTW;
+
+    // Input unit (block, row, column) of the tile; past the padded plane a clamped one, which
+    // only reaches outputs outside the image.
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(static_cast<const uint16_t*>(a.xin) + z * a.xin_ts, a.xin_bytes);
+    constexpr int kUnits = 8 * L::IPX;
+    constexpr int kIter = (kUnits + 64 * L::NW - 1) / (64 * L::NW);
+    u32x4 q[kIter];
+#pragma unroll
+    for (int j = 0; j < kIter; ++j) {
+        const int u = min(tid + j * 64 * L::NW, kUnits - 1);
+        const int cb = u / L::IPX;
+        const int r = u - cb * L::IPX;
+        const int row = r / L::IW;
+        const int py = min(oy0 + row, a.Hp - 1);
+        const int px = min(ox0 + r - row * L::IW, a.Wp - 1);
+        q[j] = load16(xr, (uint32_t)((cb * a.Hp + py) * a.Wp + px) * 16u);
+    }
+    const __amdgpu_buffer_rsrc_t w1 = make_rsrc(a.wpk1, a.wpk_bytes);
+    const __amdgpu_buffer_rsrc_t w2 = make_rsrc(a.wpk2, a.wpk_bytes);
+    const uint32_t wlane = (uint32_t)(half * 2 * 64 + lane) * 16u;
+    // This lane's channels: oc(n) .. oc(n) + 3.
+    auto oc = [&](int n) { return (half * 2 + n) * 16 + quarter * 4; };
+    float b1[2][4], b2[2][4];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            b1[n][v] = a.bias1[oc(n) + v];
+            b2[n][v] = a.bias2[oc(n) + v];
+        }
+#pragma unroll
+    for (int j = 0; j < kIter; ++j) xt[min(tid + j * 64 * L::NW, kUnits - 1)] = q[j];
+    __syncthreads();
+
+    {
+        uint32_t base[L::P1];
+#pragma unroll
+        for (int p = 0; p < L::P1; ++p) {
+            const int hp = min((group + PG * p) * 16 + (lane & 15), L::HPX - 1);
+            const int hy = hp / L::HW;
+            base[p] = (uint32_t)(quarter * L::IPX + hy * L::IW + hp - hy * L::HW) * 16u;
+        }
+        f32x4 sum[L::P1][2];
+        gemm64<L::P1, L::IPX, L::IW>(lds, base, w1, wlane, sum);
+        // t, zero outside the image (conv2's padding).
+#pragma unroll
+        for (int p = 0; p < L::P1; ++p) {
+            const int hp = (group + PG * p) * 16 + (lane & 15);
+            const int hy = min(hp, L::HPX - 1) / L::HW;
+            const int iy = oy0 - 1 + hy;
+            const int ix = ox0 - 1 + hp - hy * L::HW;
+            const bool inside = iy >= 0 && iy < a.H && ix >= 0 && ix < a.W;
+            if (hp >= L::HPX) continue;
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                float f[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) f[v] = activate(sum[p][n][v] + b1[n][v], a.act1, a.slope);
+                const Half4 h = pack4(f);
+                *reinterpret_cast<uint2*>(tt + ((oc(n) >> 3) * L::HPX + hp) * 16 + (quarter & 1) * 8) =
+                    inside ? make_uint2(h.v[0], h.v[1]) : make_uint2(0u, 0u);
+            }
+        }
+    }
+    __syncthreads();
+
+    uint32_t base[L::P2];
+#pragma unroll
+    for (int p = 0; p < L::P2; ++p)
+        base[p] = (uint32_t)(quarter * L::HPX + (group + PG * p) * L::HW + (lane & 15)) * 16u;
+    f32x4 sum[L::P2][2];
+    gemm64<L::P2, L::HPX, L::HW>(tt, base, w2, wlane, sum);
+    const uint16_t* res1 = a.res1 ? a.res1 + z * a.res1_ts : nullptr;
+    const uint16_t* res2 = a.res2 ? a.res2 + z * a.res2_ts : nullptr;
+    uint16_t* out = a.out + z * a.out_ts;
+    uint16_t* out2 = a.out2 ? a.out2 + z * a.out2_ts : nullptr;
+    const int x = ox0 + (lane & 15);
+#pragma unroll
+    for (int p = 0; p < L::P2; ++p) {
+        const int y = oy0 + group + PG * p;
+        if (y >= a.H || x >= a.W) continue;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int c = oc(n);
+            float f[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) f[v] = activate(sum[p][n][v] + b2[n][v], a.act2, a.slope);
+            if (res1 != nullptr) {
+                const Half4 h = load4(res1, a.res1_layout, c, y, x, a.H, a.W, a.Hp, a.Wp);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + f[v];
+            }
+            if (res2 != nullptr) {
+                const Half4 h = load4(res2, a.res2_layout, a.res2_coff + c, y, x, a.H, a.W, a.Hp, a.Wp);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + (float)round_f16(f[v]);
+            }
+            const Half4 h = pack4(f);
+            store4(out, a.out_layout, c, y, x, a.H, a.W, a.Hp, a.Wp, h);
+            if (out2 != nullptr) store4(out2, kLayoutCB8, c, y, x, a.H, a.W, a.Hp, a.Wp, h);
+        }
+    }
+}
+
+template <int TH, int PG>
+hipError_t launch_pair_wide(WidePairArgs a, int images, hipStream_t stream) {
+    using L = WidePair<TH, PG>;
+    a.tiles_x = (a.W + kWideTW - 1) / kWideTW;
+    a.tiles_image = (a.H + TH - 1) / TH * a.tiles_x;
+    a.tiles = images * a.tiles_image;
+    auto kernel = &conv_pair_wide_kernel<TH, PG>;
+    const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), WidePair<TH, PG>::lds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.tiles + 7) / 8 * 8)), dim3(64 * L::NW), L::lds, stream, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+static long wide_tiles(int height, int width, int images, int th) {
+    return (long)images * ((height + th - 1) / th) * ((width + kWideTW - 1) / kWideTW);
+}
+
+// Up to 256 tiles of 2 x 8 pixels the 16-pixel kernels of dcn_kernels_conv.hip run as one
+// workgroup per CU and are faster (a pair at 64x64, 256 of them: 6.7 against 7.1 us; at
+// 64x72, 288: 11.5 against 7.5). The wide kernels read and write four channels of a CB8 unit
+// at once: those tensors must be 8-byte aligned.
+bool conv_wide_chosen(int height, int width, int images, const ConvEnds& t) {
+    const auto ok = [](const void* p, int layout) { return layout != kLayoutCB8 || (uintptr_t)p % 8 == 0; };
+    return (long)images * ((height + 1) / 2) * ((width + 7) / 8) > 256 && ok(t.res1, t.res1_layout) &&
+           ok(t.res2, t.res2_layout) && ok(t.out, t.out_layout) && ok(t.out2, kLayoutCB8);
+}
+
+hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk1, const float* bias1,
+                                    int act1, const void* wpk2, const float* bias2, int act2, float slope,
+                                    const uint16_t* res1, int res1_layout, const uint16_t* res2, int res2_layout,
+                                    uint16_t* out, int out_layout, hipStream_t stream, int res2_coff,
+                                    const ConvBatch& batch, uint16_t* out2_cb8) {
+    WidePairArgs a{};
+    a.xin = x_cb8;
+    a.wpk1 = wpk1;
+    a.wpk2 = wpk2;
+    a.bias1 = bias1;
+    a.bias2 = bias2;
+    a.res1 = res1;
+    a.res2 = res2;
+    a.out = out;
+    a.out2 = out2_cb8;
+    a.act1 = act1;
+    a.act2 = act2;
+    a.slope = slope;
+    a.res1_layout = res1_layout;
+    a.res2_layout = res2_layout;
+    a.out_layout = out_layout;
+    a.res2_coff = res2_coff;
+    a.xin_ts = batch.x;
+    a.res1_ts = batch.res1;
+    a.res2_ts = batch.res2;
+    a.out_ts = batch.out;
+    a.out2_ts = batch.out2;
+    a.H = g.h;
+    a.W = g.w;
+    a.Hp = g.h + 2 * kPad;
+    a.Wp = g.w + 2 * kPad;
+    a.xin_bytes = (uint32_t)((size_t)g.cb * a.Hp * a.Wp * 16);
+    a.wpk_bytes = (uint32_t)conv_packed_bytes(g);
+    // The smallest tile whose workgroups fit the 256 CUs at once, else the largest: a round of
+    // workgroups costs mostly its latency, and beyond one round the halo counts. Measured
+    // us at TH 2 / 4 / 8 / 16: 90x91 (270 tiles of 2 rows, 138 of 4) 9.2 / 8.7 / 10.0 / 15.0,
+    // 180x320 (240 of 16) 29.1 / 28.4 / 21.0 / 17.3.
+    const auto fits = [&](int th) { return wide_tiles(g.h, g.w, batch.images, th) <= 256; };
+    if (fits(2)) return launch_pair_wide<2, 2>(a, batch.images, stream);
+    if (fits(4)) return launch_pair_wide<4, 4>(a, batch.images, stream);
+    if (fits(8)) return launch_pair_wide<8, 4>(a, batch.images, stream);
+    return launch_pair_wide<16, 4>(a, batch.images, stream);
+}
+
+}  // namespace dcn

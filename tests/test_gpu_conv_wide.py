@@ -1,0 +1,85 @@
+"""GPU tests of the large-tile body convolutions (many pixels): the same bits as the
+16-pixel-tile kernels, which take every call whose CB8 tensors are not 8-byte aligned."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import body_reference as br
+
+pytestmark = pytest.mark.gpu
+
+NCHW, CB8 = 0, 1
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+
+    return t
+
+
+def _dev(torch, a):
+    return torch.from_numpy(np.ascontiguousarray(np.asarray(a, np.float16)).view(np.int16)).cuda()
+
+
+def _placed(torch, elems, shift):
+    """A zeroed device tensor of `elems` halves, `shift` halves past an aligned address."""
+    return torch.zeros(elems + 8, dtype=torch.int16, device="cuda")[shift:shift + elems]
+
+
+def _operand(torch, a, shift):
+    t = _placed(torch, a.size, shift)
+    t.copy_(_dev(torch, a.ravel()))
+    return t
+
+
+# Height, width: one to sixteen rows per tile by the number of tiles, with partial tiles on
+# both sides and maps narrower than a tile.
+SIZES = [(33, 129), (90, 91), (47, 331), (131, 133), (181, 317), (1033, 3), (5, 1500)]
+
+
+@pytest.mark.parametrize("h,w", SIZES, ids=lambda v: str(v))
+@pytest.mark.parametrize("acts,layouts,residuals", [((2, 0), (CB8, CB8, CB8), 1), ((1, 1), (CB8, CB8, CB8), 0),
+                                                    ((2, 0), (CB8, CB8, NCHW), 2), ((0, 2), (NCHW, NCHW, NCHW), 2),
+                                                    ((1, 0), (NCHW, CB8, CB8), 2)])
+def test_wide_pair_same_bits(gpu_ctx, torch, h, w, acts, layouts, residuals):
+    rng = np.random.default_rng(h * 1000 + w + 7 * acts[0])
+    plane = h * w
+    print("case: wide pair", h, w, acts, layouts, residuals, flush=True)
+    f16 = lambda *s, std=1.0: br.f16(rng.normal(0, std, s))  # noqa: E731
+    x = f16(64, h, w)
+    x[3, h // 2, w // 2], x[9, 0, 0], x[20, h - 1, w - 1] = np.inf, np.nan, -np.inf
+    convs = [gpu_ctx.conv3x3(64, 64, h, w, _dev(torch, f16(64, 64, 3, 3, std=0.04)), _dev(torch, f16(64, std=0.1)))
+             for _ in range(2)]
+    xd = _dev(torch, br.to_cb8(x, 64, h, w))
+    res = [f16(64, h, w) for _ in range(2)]
+
+    def run(shift):
+        r = [_operand(torch, br.to_cb8(a, 64, h, w) if l == CB8 else a, shift if l == CB8 else 0) if i < residuals
+             else None for i, (a, l) in enumerate(zip(res, layouts[:2]))]
+        out = _placed(torch, 8 * (h + 4) * (w + 4) * 8 if layouts[2] == CB8 else 64 * plane,
+                      shift if layouts[2] == CB8 else 0)
+        convs[0].run_pair_dev(convs[1], xd, out, layouts[2], activation1=acts[0], activation2=acts[1], res1=r[0],
+                              res1_layout=layouts[0], res2=r[1], res2_layout=layouts[1])
+        torch.cuda.synchronize()
+        return out.cpu().numpy().view(np.uint16).copy()
+
+    got = run(0)
+    if CB8 in layouts[:residuals] + layouts[2:]:
+        want = run(1)
+    else:  # no CB8 tensor to misalign: two single-conv calls
+        mid = _placed(torch, 8 * (h + 4) * (w + 4) * 8, 1)
+        out = _placed(torch, 64 * plane, 0)
+        r = [_dev(torch, a) for a in res]
+        convs[0].run_dev(xd, mid, CB8, activation=acts[0])
+        mid2 = mid.clone()
+        convs[1].run_dev(mid2, out, NCHW, activation=acts[1], res1=r[0], res1_layout=NCHW, res2=r[1], res2_layout=NCHW)
+        torch.cuda.synchronize()
+        want = out.cpu().numpy().view(np.uint16).copy()
+    for c in convs:
+        c.free()
+    a, b = got.view(np.float16), want.view(np.float16)
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    assert np.array_equal(got[~np.isnan(b)], want[~np.isnan(b)])
+    assert np.isfinite(a).mean() > 0.9
