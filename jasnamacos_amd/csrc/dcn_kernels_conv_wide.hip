@@ -314,6 +314,193 @@ hipError_t launch_pair_wide(WidePairArgs a, int images, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// One 3x3 conv of 8 * CB input channels (conv3x3_kernel's contract) on a TH x 16 output tile:
+// the tile's input (one pixel more on each side, all channels: K runs over taps outside and
+// channels inside) comes into LDS by DMA. Over 16 maps of 64x64, 320 -> 64 channels 80.5 ->
+// 31.8 us (760 TFLOP/s), 196 -> 64 37.2 -> 19.1 us; 180x320 64 -> 432 130 -> 39.9 us. Each of the
+// four waves of a workgroup multiplies half of the rows by half of the channels; what bounds it
+// is the weight fragments, 2 KB per wave and K-step through the L1 for 4 or 8 products.
+struct WideConvArgs {
+    const void* xin;
+    const void* wpk;
+    const float* bias;
+    const uint16_t* res1;
+    const uint16_t* res2;
+    uint16_t* out;
+    uint32_t xin_bytes, wpk_bytes;
+    int act;
+    float slope;
+    int res1_layout, res2_layout, out_layout, res2_coff;
+    int H, W, Hp, Wp, Cout, NBT, tiles_x, tiles_image, tiles;
+    long xin_ts, res1_ts, res2_ts, out_ts;
+};
+
+template <int CB, int TH, int PG>
+struct WideConv {
+    static constexpr int NW = 2 * PG;
+    static constexpr int IW = kWideTW + 2, IPX = (TH + 2) * IW;
+    static constexpr int P = TH / PG;
+    static constexpr int KB = 9 * CB, KSTEPS = (KB + 3) / 4;
+    static constexpr int UNITS = (CB * IPX + 63) / 64 * 64;  // whole waves of DMA
+    static constexpr size_t lds = (size_t)UNITS * 16;
+};
+
+template <int CB, int TH, int PG>
+__global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_kernel(WideConvArgs a) {
+    using L = WideConv<CB, TH, PG>;
+    constexpr int P = L::P;
+    constexpr int D = P == 4 ? 4 : 6;  // K-steps of weights in flight
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = wave >> 1;
+    const int half = wave & 1;
+    const int quarter = lane >> 4;
+
+    const int per_xcd = (a.tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= a.tiles) return;  // whole workgroup, before any barrier
+    const int z = tile / a.tiles_image;
+    const int ti = tile - z * a.tiles_image;
+    const int ty = ti / a.tiles_x;
+    const int oy0 = ty * TH;
+    const int ox0 = (ti - ty * a.tiles_x) * kWideTW;
+    const int chunk = blockIdx.y;
+
+    // Input unit u = (block, row, column) of the tile, from one pixel up and left of it; past
+    // the padded plane a clamped one, which only reaches outputs outside the image.
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(static_cast<const uint16_t*>(a.xin) + z * a.xin_ts, a.xin_bytes);
+    for (int u0 = wave * 64; u0 < L::UNITS; u0 += 64 * L::NW) {
+        const int u = min(u0 + lane, CB * L::IPX - 1);
+        const int cb = u / L::IPX;
+        const int r = u - cb * L::IPX;
+        const int row = r / L::IW;
+        const int py = min(oy0 + row + kPad - 1, a.Hp - 1);
+        const int px = min(ox0 + r - row * L::IW + kPad - 1, a.Wp - 1);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(lds + u0 * 16), 16,
+                                                 (int)((uint32_t)((cb * a.Hp + py) * a.Wp + px) * 16u), 0, 0, 0);
+    }
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.wpk, a.wpk_bytes);
+    uint32_t wlane = (uint32_t)((chunk * 4 + half * 2) * 64 + lane) * 16u;
+    auto oc = [&](int n) { return chunk * 64 + (half * 2 + n) * 16 + quarter * 4; };
+    h8 B[D][2];
+    auto load_weights = [&](int s) {
+        __asm__ volatile("" : "+v"(wlane));  // requested here and not earlier
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+            B[s % D][n] = __builtin_bit_cast(h8, load16(wr, wlane, (uint32_t)(s * a.NBT + n) * 1024u));
+    };
+    float bias[2][4];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) bias[n][v] = a.bias[min(oc(n) + v, a.Cout - 1)];
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's copies (the compiler does not track them)
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < D - 1 && s < L::KSTEPS; ++s) load_weights(s);
+
+    // Byte address of K-block 4 s + quarter's unit of each row; K-blocks of two taps in one
+    // step (CB not a multiple of 4) move the lanes of the later one.
+    uint32_t base[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+        base[p] = (uint32_t)(quarter * L::IPX + (group + PG * p) * L::IW + (lane & 15)) * 16u;
+    auto unit = [](int kb) { return kb % CB * L::IPX + kb / CB / 3 * L::IW + kb / CB % 3; };
+    h8 X[2][P];
+    auto load_pixels = [&](int s) {
+        const int kb = 4 * s;
+        const int wrap = CB - kb % CB;  // lanes of this quarter and later are in the next tap
+        const uint32_t off = (uint32_t)unit(kb) * 16u;
+        uint32_t more = 0;
+        if (wrap < 4 && kb + wrap < L::KB)
+            more = quarter >= wrap ? (uint32_t)(unit(kb + wrap) - unit(kb) - wrap * L::IPX) * 16u : 0u;
+#pragma unroll
+        for (int p = 0; p < P; ++p) X[s & 1][p] = *reinterpret_cast<const h8*>(lds + (base[p] + off + more));
+        if (kb + 4 > L::KB) {
+            // Padding K-blocks multiply zero weights; zero pixels keep a non-finite input from
+            // turning 0 * inf into NaN there.
+            const h8 zero = __builtin_bit_cast(h8, u32x4{0u, 0u, 0u, 0u});
+#pragma unroll
+            for (int p = 0; p < P; ++p) X[s & 1][p] = kb + quarter < L::KB ? X[s & 1][p] : zero;
+        }
+    };
+    f32x4 acc[P][2], sum[P][2];
+    load_pixels(0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        constexpr int K = L::KSTEPS;
+        const int s0 = r * K / 8, s1 = (r + 1) * K / 8;
+#pragma unroll
+        for (int s = s0; s < s1; ++s) {
+            if (s + D - 1 < K) load_weights(s + D - 1);
+            if (s + 1 < K) load_pixels(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+                    acc[p][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(B[s % D][n], X[s & 1][p],
+                                                                       s == s0 ? f32x4{} : acc[p][n], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                if (r == 0)
+                    sum[p][n] = acc[p][n];
+                else
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sum[p][n][v] = sum[p][n][v] + acc[p][n][v];
+                __asm__ volatile("" : "+v"(sum[p][n]));
+            }
+    }
+
+    const uint16_t* res1 = a.res1 ? a.res1 + z * a.res1_ts : nullptr;
+    const uint16_t* res2 = a.res2 ? a.res2 + z * a.res2_ts : nullptr;
+    uint16_t* out = a.out + z * a.out_ts;
+    const int x = ox0 + (lane & 15);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int y = oy0 + group + PG * p;
+        if (y >= a.H || x >= a.W) continue;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int c = oc(n);
+            if (c >= a.Cout) continue;
+            float f[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) f[v] = activate(sum[p][n][v] + bias[n][v], a.act, a.slope);
+            if (res1 != nullptr) {
+                const Half4 h = load4(res1, a.res1_layout, c, y, x, a.H, a.W, a.Hp, a.Wp);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + f[v];
+            }
+            if (res2 != nullptr) {
+                const Half4 h = load4(res2, a.res2_layout, a.res2_coff + c, y, x, a.H, a.W, a.Hp, a.Wp);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + (float)round_f16(f[v]);
+            }
+            store4(out, a.out_layout, c, y, x, a.H, a.W, a.Hp, a.Wp, pack4(f));
+        }
+    }
+}
+
+template <int CB, int TH, int PG>
+hipError_t launch_wide_as(WideConvArgs a, int images, int chunks, hipStream_t stream) {
+    using L = WideConv<CB, TH, PG>;
+    a.tiles_x = (a.W + kWideTW - 1) / kWideTW;
+    a.tiles_image = (a.H + TH - 1) / TH * a.tiles_x;
+    a.tiles = images * a.tiles_image;
+    auto kernel = &conv_wide_kernel<CB, TH, PG>;
+    const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), L::lds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.tiles + 7) / 8 * 8), (unsigned)chunks), dim3(64 * L::NW), L::lds, stream, a);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 static long wide_tiles(int height, int width, int images, int th) {
@@ -322,12 +509,17 @@ static long wide_tiles(int height, int width, int images, int th) {
 
 // Up to 256 tiles of 2 x 8 pixels the 16-pixel kernels of dcn_kernels_conv.hip run as one
 // workgroup per CU and are faster (a pair at 64x64, 256 of them: 6.7 against 7.1 us; at
-// 64x72, 288: 11.5 against 7.5). The wide kernels read and write four channels of a CB8 unit
+// 64x72, 288: 11.5 against 7.5; 320 -> 64 there 10.7 against 10.0). The wide kernels read and write four channels of a CB8 unit
 // at once: those tensors must be 8-byte aligned.
-bool conv_wide_chosen(int height, int width, int images, const ConvEnds& t) {
+bool conv_wide_chosen(int height, int width, int images, const ConvEnds& t, int chunks) {
     const auto ok = [](const void* p, int layout) { return layout != kLayoutCB8 || (uintptr_t)p % 8 == 0; };
-    return (long)images * ((height + 1) / 2) * ((width + 7) / 8) > 256 && ok(t.res1, t.res1_layout) &&
+    return (long)images * ((height + 1) / 2) * ((width + 7) / 8) * chunks > 256 && ok(t.res1, t.res1_layout) &&
            ok(t.res2, t.res2_layout) && ok(t.out, t.out_layout) && ok(t.out2, kLayoutCB8);
+}
+
+bool conv_wide_supported(const ConvGeometry& g) {
+    const int cb = g.cb;
+    return (cb == 8 || cb == 16 || cb == 24 || cb == 25 || cb == 32 || cb == 40) && g.cout % 4 == 0;
 }
 
 hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk1, const float* bias1,
@@ -372,6 +564,61 @@ hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, co
     if (fits(4)) return launch_pair_wide<4, 4>(a, batch.images, stream);
     if (fits(8)) return launch_pair_wide<8, 4>(a, batch.images, stream);
     return launch_pair_wide<16, 4>(a, batch.images, stream);
+}
+
+namespace {
+
+// Tiles of 4 rows, two or more workgroups per CU; of 8 rows (half the weight traffic per pixel)
+// where there are more than 256 of those and the channels leave room for two in a CU's LDS.
+// us at TH 4 / 8: 256x256 128 -> 64 15.7 / 13.7, 196 -> 64 21.3 / 19.1, 320 -> 64 31.8 / 33.2;
+// 128x128 (128 tiles of 8 rows) 128 -> 64 6.3 / 8.8, 64 -> 432 14.8 / 17.3.
+template <int CB>
+hipError_t launch_wide_cb(const WideConvArgs& a, int images, int chunks, hipStream_t stream) {
+    if constexpr (CB <= 25)
+        if (wide_tiles(a.H, a.W, images, 8) > 256) return launch_wide_as<CB, 8, 2>(a, images, chunks, stream);
+    return launch_wide_as<CB, 4, 2>(a, images, chunks, stream);
+}
+
+}  // namespace
+
+hipError_t launch_conv3x3_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk, const float* bias, int act,
+                               float slope, const uint16_t* res1, int res1_layout, const uint16_t* res2,
+                               int res2_layout, uint16_t* out, int out_layout, hipStream_t stream, int res2_coff,
+                               const ConvBatch& batch) {
+    WideConvArgs a{};
+    a.xin = x_cb8;
+    a.wpk = wpk;
+    a.bias = bias;
+    a.res1 = res1;
+    a.res2 = res2;
+    a.out = out;
+    a.act = act;
+    a.slope = slope;
+    a.res1_layout = res1_layout;
+    a.res2_layout = res2_layout;
+    a.out_layout = out_layout;
+    a.res2_coff = res2_coff;
+    a.xin_ts = batch.x;
+    a.res1_ts = batch.res1;
+    a.res2_ts = batch.res2;
+    a.out_ts = batch.out;
+    a.H = g.h;
+    a.W = g.w;
+    a.Hp = g.h + 2 * kPad;
+    a.Wp = g.w + 2 * kPad;
+    a.Cout = g.cout;
+    a.NBT = g.nbt;
+    a.xin_bytes = (uint32_t)((size_t)g.cb * a.Hp * a.Wp * 16);
+    a.wpk_bytes = (uint32_t)conv_packed_bytes(g);
+    switch (g.cb) {
+        case 8: return launch_wide_cb<8>(a, batch.images, g.chunks, stream);
+        case 16: return launch_wide_cb<16>(a, batch.images, g.chunks, stream);
+        case 24: return launch_wide_cb<24>(a, batch.images, g.chunks, stream);
+        case 25: return launch_wide_cb<25>(a, batch.images, g.chunks, stream);
+        case 32: return launch_wide_cb<32>(a, batch.images, g.chunks, stream);
+        case 40: return launch_wide_cb<40>(a, batch.images, g.chunks, stream);
+    }
+    return hipErrorInvalidValue;
 }
 
 }  // namespace dcn

@@ -83,3 +83,38 @@ def test_wide_pair_same_bits(gpu_ctx, torch, h, w, acts, layouts, residuals):
     assert np.array_equal(np.isnan(a), np.isnan(b))
     assert np.array_equal(got[~np.isnan(b)], want[~np.isnan(b)])
     assert np.isfinite(a).mean() > 0.9
+
+
+# (cin, cout): each channel-block count of the kernel, whole and partial last output chunk
+CHANNELS = [(64, 64), (128, 64), (192, 20), (196, 64), (256, 64), (320, 64), (61, 432)]
+
+
+@pytest.mark.parametrize("cin,cout", CHANNELS, ids=lambda v: str(v))
+@pytest.mark.parametrize("h,w,act,residuals,layout", [(67, 131, 1, 0, CB8), (90, 401, 2, 2, CB8), (5, 1500, 0, 1, NCHW)])
+def test_wide_conv_same_bits(gpu_ctx, torch, cin, cout, h, w, act, residuals, layout):
+    """One conv on tiles of 4 and 8 rows against the 16-pixel-tile kernel."""
+    rng = np.random.default_rng(cin * 7 + cout + h)
+    print("case: wide conv", cin, cout, h, w, act, residuals, layout, flush=True)
+    f16 = lambda *s, std=1.0: br.f16(rng.normal(0, std, s))  # noqa: E731
+    x = f16(cin, h, w)
+    x[cin - 1, 0, 0], x[0, h - 1, w // 2] = np.inf, np.nan
+    conv = gpu_ctx.conv3x3(cin, cout, h, w, _dev(torch, f16(cout, cin, 3, 3, std=0.04)), _dev(torch, f16(cout, std=0.1)))
+    xd = _dev(torch, br.to_cb8(x, cin, h, w))
+    res = [f16(cout, h, w) for _ in range(2)]
+    res_l = [CB8, NCHW]
+    cb = (cout + 7) // 8
+
+    def run(shift):
+        r = [_operand(torch, br.to_cb8(a, cout, h, w) if l == CB8 else a, shift if l == CB8 else 0) if i < residuals
+             else None for i, (a, l) in enumerate(zip(res, res_l))]
+        out = _placed(torch, cb * 8 * (h + 4) * (w + 4) if layout == CB8 else cout * h * w, shift if layout == CB8 else 0)
+        conv.run_dev(xd, out, layout, activation=act, res1=r[0], res1_layout=CB8, res2=r[1], res2_layout=NCHW)
+        torch.cuda.synchronize()
+        return out.cpu().numpy().view(np.uint16).copy()
+
+    got, want = run(0), run(1)
+    conv.free()
+    a, b = got.view(np.float16), want.view(np.float16)
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    assert np.array_equal(got[~np.isnan(b)], want[~np.isnan(b)])
+    assert np.isfinite(a).mean() > 0.9
