@@ -279,6 +279,11 @@ hipError_t launch_convk_prepack(const ConvKGeometry& g, const uint16_t* w, const
 hipError_t launch_convk(const ConvKGeometry& g, int batch, int pad, const void* x_cb8, const void* wpk,
                         const float* bias, int act, const uint16_t* base, uint16_t* out, int out_cb8,
                         hipStream_t stream);
+// launch_convk on larger tiles (dcn_kernels_conv_wide.hip), run where convk_wide_chosen.
+bool convk_wide_chosen(const ConvKGeometry& g, int batch, const uint16_t* out, int out_cb8);
+hipError_t launch_convk_wide(const ConvKGeometry& g, int batch, int pad, const void* x_cb8, const void* wpk,
+                             const float* bias, int act, const uint16_t* base, uint16_t* out, int out_cb8,
+                             hipStream_t stream);
 hipError_t launch_bicubic_quarter(const uint16_t* in, uint16_t* out, int channels, int height, int width,
                                   hipStream_t stream);
 // Pyramids of `count` RGB frames (frame 0, frame 1, frame f >= 2 at frame0 + f * stride):

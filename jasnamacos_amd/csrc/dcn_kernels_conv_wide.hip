@@ -51,33 +51,39 @@ struct Half4 {
 __device__ __forceinline__ float half_at(const Half4& h, int i) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)(h.v[i >> 1] >> (16 * (i & 1))));
 }
-__device__ __forceinline__ Half4 load4(const uint16_t* t, int layout, int c, int y, int x, int H, int W, int Hp, int Wp) {
+struct Place {
+    int H, W, pad;  // image, and border of a CB8 tensor
+};
+// The first `live` of them of an NCHW tensor (a CB8 one holds all four).
+__device__ __forceinline__ Half4 load4(const uint16_t* t, int layout, int c, int y, int x, const Place& a, int live = 4) {
     Half4 r;
     if (layout == kLayoutCB8) {
-        const uint2 u = *reinterpret_cast<const uint2*>(t + ((size_t)((c >> 3) * Hp + y + kPad) * Wp + x + kPad) * 8 + (c & 7));
+        const size_t unit = ((size_t)(c >> 3) * (a.H + 2 * a.pad) + y + a.pad) * (a.W + 2 * a.pad) + x + a.pad;
+        const uint2 u = *reinterpret_cast<const uint2*>(t + unit * 8 + (c & 7));
         r.v[0] = u.x;
         r.v[1] = u.y;
     } else {
-        const size_t plane = (size_t)H * W;
-        const uint16_t* p = t + (size_t)c * plane + (size_t)y * W + x;
-        const uint32_t a = p[0], b = p[plane], d = p[2 * plane], e = p[3 * plane];
-        r.v[0] = a | (b << 16);
-        r.v[1] = d | (e << 16);
+        const size_t plane = (size_t)a.H * a.W;
+        const uint16_t* p = t + (size_t)c * plane + (size_t)y * a.W + x;
+        const uint32_t h0 = p[0], h1 = live > 1 ? p[plane] : 0u;
+        const uint32_t h2 = live > 2 ? p[2 * plane] : 0u, h3 = live > 3 ? p[3 * plane] : 0u;
+        r.v[0] = h0 | (h1 << 16);
+        r.v[1] = h2 | (h3 << 16);
     }
     return r;
 }
-__device__ __forceinline__ void store4(uint16_t* t, int layout, int c, int y, int x, int H, int W, int Hp, int Wp,
-                                       const Half4& h) {
+__device__ __forceinline__ void store4(uint16_t* t, int layout, int c, int y, int x, const Place& a, const Half4& h,
+                                       int live = 4) {
     if (layout == kLayoutCB8) {
-        *reinterpret_cast<uint2*>(t + ((size_t)((c >> 3) * Hp + y + kPad) * Wp + x + kPad) * 8 + (c & 7)) =
-            make_uint2(h.v[0], h.v[1]);
+        const size_t unit = ((size_t)(c >> 3) * (a.H + 2 * a.pad) + y + a.pad) * (a.W + 2 * a.pad) + x + a.pad;
+        *reinterpret_cast<uint2*>(t + unit * 8 + (c & 7)) = make_uint2(h.v[0], h.v[1]);
     } else {
-        const size_t plane = (size_t)H * W;
-        uint16_t* p = t + (size_t)c * plane + (size_t)y * W + x;
+        const size_t plane = (size_t)a.H * a.W;
+        uint16_t* p = t + (size_t)c * plane + (size_t)y * a.W + x;
         p[0] = (uint16_t)h.v[0];
-        p[plane] = (uint16_t)(h.v[0] >> 16);
-        p[2 * plane] = (uint16_t)h.v[1];
-        p[3 * plane] = (uint16_t)(h.v[1] >> 16);
+        if (live > 1) p[plane] = (uint16_t)(h.v[0] >> 16);
+        if (live > 2) p[2 * plane] = (uint16_t)h.v[1];
+        if (live > 3) p[3 * plane] = (uint16_t)(h.v[1] >> 16);
     }
 }
 __device__ __forceinline__ Half4 pack4(const float (&f)[4]) {
@@ -274,6 +280,7 @@ __global__ __launch_bounds__((64 * WidePair<TH, PG>::NW)) void conv_pair_wide_ke
     uint16_t* out = a.out + z * a.out_ts;
     uint16_t* out2 = a.out2 ? a.out2 + z * a.out2_ts : nullptr;
     const int x = ox0 + (lane & 15);
+    const Place place{a.H, a.W, kPad};
 #pragma unroll
     for (int p = 0; p < L::P2; ++p) {
         const int y = oy0 + group + PG * p;
@@ -285,18 +292,18 @@ __global__ __launch_bounds__((64 * WidePair<TH, PG>::NW)) void conv_pair_wide_ke
 #pragma unroll
             for (int v = 0; v < 4; ++v) f[v] = activate(sum[p][n][v] + b2[n][v], a.act2, a.slope);
             if (res1 != nullptr) {
-                const Half4 h = load4(res1, a.res1_layout, c, y, x, a.H, a.W, a.Hp, a.Wp);
+                const Half4 h = load4(res1, a.res1_layout, c, y, x, place);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + f[v];
             }
             if (res2 != nullptr) {
-                const Half4 h = load4(res2, a.res2_layout, a.res2_coff + c, y, x, a.H, a.W, a.Hp, a.Wp);
+                const Half4 h = load4(res2, a.res2_layout, a.res2_coff + c, y, x, place);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + (float)round_f16(f[v]);
             }
             const Half4 h = pack4(f);
-            store4(out, a.out_layout, c, y, x, a.H, a.W, a.Hp, a.Wp, h);
-            if (out2 != nullptr) store4(out2, kLayoutCB8, c, y, x, a.H, a.W, a.Hp, a.Wp, h);
+            store4(out, a.out_layout, c, y, x, place, h);
+            if (out2 != nullptr) store4(out2, kLayoutCB8, c, y, x, place, h);
         }
     }
 }
@@ -314,12 +321,15 @@ hipError_t launch_pair_wide(WidePairArgs a, int images, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// One 3x3 conv of 8 * CB input channels (conv3x3_kernel's contract) on a TH x 16 output tile:
-// the tile's input (one pixel more on each side, all channels: K runs over taps outside and
-// channels inside) comes into LDS by DMA. Over 16 maps of 64x64, 320 -> 64 channels 80.5 ->
-// 31.8 us (760 TFLOP/s), 196 -> 64 37.2 -> 19.1 us; 180x320 64 -> 432 130 -> 39.9 us. Each of the
-// four waves of a workgroup multiplies half of the rows by half of the channels; what bounds it
-// is the weight fragments, 2 KB per wave and K-step through the L1 for 4 or 8 products.
+// One KS x KS conv of 8 * CB input channels (conv3x3_kernel's contract, and convk_kernel's) on a
+// TH x 16 output tile: the tile's input (KS / 2 pixels more on each side, all channels: K runs
+// over taps outside and channels inside) comes into LDS by DMA. NH * PG waves: each multiplies
+// every PG-th row by N of the NH * N 16-channel blocks.
+//
+// 3x3 over 16 maps of 64x64: 320 -> 64 channels 80.5 -> 31.8 us (760 TFLOP/s), 196 -> 64
+// 37.2 -> 19.1 us; 180x320 64 -> 432 130 -> 39.9 us. What bounds it: the weight fragments, 2 KB per
+// wave and K-step through the L1 for 4 or 8 products, and the pixel fragments, half a KB
+// of LDS per product with N = 2 (as long as the product takes), one with N = 1.
 struct WideConvArgs {
     const void* xin;
     const void* wpk;
@@ -331,32 +341,40 @@ struct WideConvArgs {
     int act;
     float slope;
     int res1_layout, res2_layout, out_layout, res2_coff;
-    int H, W, Hp, Wp, Cout, NBT, tiles_x, tiles_image, tiles;
+    int H, W, pad, Cout, NBT, tiles_x, tiles_image, tiles;  // pad: border of every CB8 tensor
     long xin_ts, res1_ts, res2_ts, out_ts;
 };
 
-template <int CB, int TH, int PG>
+template <int KS, int CB, int NH, int N, int TH, int PG>
 struct WideConv {
-    static constexpr int NW = 2 * PG;
-    static constexpr int IW = kWideTW + 2, IPX = (TH + 2) * IW;
+    static constexpr int NW = NH * PG;
+    static constexpr int IW = kWideTW + KS - 1, IPX = (TH + KS - 1) * IW;
     static constexpr int P = TH / PG;
-    static constexpr int KB = 9 * CB, KSTEPS = (KB + 3) / 4;
+    static constexpr int KB = KS * KS * CB, KSTEPS = (KB + 3) / 4;
     static constexpr int UNITS = (CB * IPX + 63) / 64 * 64;  // whole waves of DMA
     static constexpr size_t lds = (size_t)UNITS * 16;
+    // LDS unit of K-block kb of the pixel whose tap (0, 0) is unit 0 (a padding K-block: the
+    // last one's), and lane quarter q's at K-block 0.
+    static constexpr int unit(int kb) {
+        const int k = kb < KB ? kb : KB - 1;
+        return k % CB * IPX + k / CB / KS * IW + k / CB % KS;
+    }
+    static constexpr int first(int q) { return CB >= 4 ? q * IPX : q % CB * IPX + q / CB; }
 };
 
-template <int CB, int TH, int PG>
-__global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_kernel(WideConvArgs a) {
-    using L = WideConv<CB, TH, PG>;
+template <int KS, int CB, int NH, int N, int TH, int PG>
+__global__ __launch_bounds__((64 * NH * PG)) void conv_wide_kernel(WideConvArgs a) {
+    using L = WideConv<KS, CB, NH, N, TH, PG>;
     constexpr int P = L::P;
-    constexpr int D = P == 4 ? 4 : 6;  // K-steps of weights in flight
+    constexpr int D = P == 4 ? 4 : P == 2 ? 6 : 8;  // K-steps of weights in flight
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = wave >> 1;
-    const int half = wave & 1;
+    const int group = wave / NH;
+    const int half = wave % NH;
     const int quarter = lane >> 4;
+    const int Hp = a.H + 2 * a.pad, Wp = a.W + 2 * a.pad;
 
     const int per_xcd = (a.tiles + 7) / 8;
     const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -368,32 +386,32 @@ __global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_ker
     const int ox0 = (ti - ty * a.tiles_x) * kWideTW;
     const int chunk = blockIdx.y;
 
-    // Input unit u = (block, row, column) of the tile, from one pixel up and left of it; past
-    // the padded plane a clamped one, which only reaches outputs outside the image.
+    // Input unit u = (block, row, column) of the tile, from KS / 2 pixels up and left of it;
+    // past the padded plane a clamped one, which only reaches outputs outside the image.
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(static_cast<const uint16_t*>(a.xin) + z * a.xin_ts, a.xin_bytes);
     for (int u0 = wave * 64; u0 < L::UNITS; u0 += 64 * L::NW) {
         const int u = min(u0 + lane, CB * L::IPX - 1);
         const int cb = u / L::IPX;
         const int r = u - cb * L::IPX;
         const int row = r / L::IW;
-        const int py = min(oy0 + row + kPad - 1, a.Hp - 1);
-        const int px = min(ox0 + r - row * L::IW + kPad - 1, a.Wp - 1);
+        const int py = min(oy0 + row + a.pad - KS / 2, Hp - 1);
+        const int px = min(ox0 + r - row * L::IW + a.pad - KS / 2, Wp - 1);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(lds + u0 * 16), 16,
-                                                 (int)((uint32_t)((cb * a.Hp + py) * a.Wp + px) * 16u), 0, 0, 0);
+                                                 (int)((uint32_t)((cb * Hp + py) * Wp + px) * 16u), 0, 0, 0);
     }
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.wpk, a.wpk_bytes);
-    uint32_t wlane = (uint32_t)((chunk * 4 + half * 2) * 64 + lane) * 16u;
-    auto oc = [&](int n) { return chunk * 64 + (half * 2 + n) * 16 + quarter * 4; };
-    h8 B[D][2];
+    uint32_t wlane = (uint32_t)(((chunk * NH + half) * N) * 64 + lane) * 16u;
+    auto oc = [&](int n) { return ((chunk * NH + half) * N + n) * 16 + quarter * 4; };
+    h8 B[D][N];
     auto load_weights = [&](int s) {
         __asm__ volatile("" : "+v"(wlane));  // requested here and not earlier
 #pragma unroll
-        for (int n = 0; n < 2; ++n)
+        for (int n = 0; n < N; ++n)
             B[s % D][n] = __builtin_bit_cast(h8, load16(wr, wlane, (uint32_t)(s * a.NBT + n) * 1024u));
     };
-    float bias[2][4];
+    float bias[N][4];
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
+    for (int n = 0; n < N; ++n)
 #pragma unroll
         for (int v = 0; v < 4; ++v) bias[n][v] = a.bias[min(oc(n) + v, a.Cout - 1)];
     __builtin_amdgcn_s_waitcnt(0);  // this wave's copies (the compiler does not track them)
@@ -401,21 +419,25 @@ __global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_ker
 #pragma unroll
     for (int s = 0; s < D - 1 && s < L::KSTEPS; ++s) load_weights(s);
 
-    // Byte address of K-block 4 s + quarter's unit of each row; K-blocks of two taps in one
-    // step (CB not a multiple of 4) move the lanes of the later one.
+    // Byte address of this lane's unit of each row at K-block quarter; later steps add the
+    // same offset in every lane, except where a step's K-blocks cross a tap or a tap row.
     uint32_t base[P];
 #pragma unroll
-    for (int p = 0; p < P; ++p)
-        base[p] = (uint32_t)(quarter * L::IPX + (group + PG * p) * L::IW + (lane & 15)) * 16u;
-    auto unit = [](int kb) { return kb % CB * L::IPX + kb / CB / 3 * L::IW + kb / CB % 3; };
+    for (int p = 0; p < P; ++p) {
+        const int q0 = CB >= 4 ? quarter * L::IPX : quarter % CB * L::IPX + quarter / CB;
+        base[p] = (uint32_t)(q0 + (group + PG * p) * L::IW + (lane & 15)) * 16u;
+    }
     h8 X[2][P];
     auto load_pixels = [&](int s) {
         const int kb = 4 * s;
-        const int wrap = CB - kb % CB;  // lanes of this quarter and later are in the next tap
-        const uint32_t off = (uint32_t)unit(kb) * 16u;
+        const uint32_t off = (uint32_t)L::unit(kb) * 16u;
         uint32_t more = 0;
-        if (wrap < 4 && kb + wrap < L::KB)
-            more = quarter >= wrap ? (uint32_t)(unit(kb + wrap) - unit(kb) - wrap * L::IPX) * 16u : 0u;
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+            const int d = L::unit(kb + q) - L::unit(kb) - L::first(q);
+            const int before = q == 1 ? 0 : L::unit(kb + q - 1) - L::unit(kb) - L::first(q - 1);
+            if (d != before) more = quarter >= q ? (uint32_t)(d * 16) : more;
+        }
 #pragma unroll
         for (int p = 0; p < P; ++p) X[s & 1][p] = *reinterpret_cast<const h8*>(lds + (base[p] + off + more));
         if (kb + 4 > L::KB) {
@@ -426,7 +448,7 @@ __global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_ker
             for (int p = 0; p < P; ++p) X[s & 1][p] = kb + quarter < L::KB ? X[s & 1][p] : zero;
         }
     };
-    f32x4 acc[P][2], sum[P][2];
+    f32x4 acc[P][N], sum[P][N];
     load_pixels(0);
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
@@ -440,7 +462,7 @@ __global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_ker
 #pragma unroll
             for (int p = 0; p < P; ++p)
 #pragma unroll
-                for (int n = 0; n < 2; ++n)
+                for (int n = 0; n < N; ++n)
                     acc[p][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(B[s % D][n], X[s & 1][p],
                                                                        s == s0 ? f32x4{} : acc[p][n], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
@@ -448,7 +470,7 @@ __global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_ker
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
-            for (int n = 0; n < 2; ++n) {
+            for (int n = 0; n < N; ++n) {
                 if (r == 0)
                     sum[p][n] = acc[p][n];
                 else
@@ -462,39 +484,41 @@ __global__ __launch_bounds__((64 * WideConv<CB, TH, PG>::NW)) void conv_wide_ker
     const uint16_t* res2 = a.res2 ? a.res2 + z * a.res2_ts : nullptr;
     uint16_t* out = a.out + z * a.out_ts;
     const int x = ox0 + (lane & 15);
+    const Place place{a.H, a.W, a.pad};
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const int y = oy0 + group + PG * p;
         if (y >= a.H || x >= a.W) continue;
 #pragma unroll
-        for (int n = 0; n < 2; ++n) {
+        for (int n = 0; n < N; ++n) {
             const int c = oc(n);
             if (c >= a.Cout) continue;
+            const int live = min(4, a.Cout - c);
             float f[4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) f[v] = activate(sum[p][n][v] + bias[n][v], a.act, a.slope);
             if (res1 != nullptr) {
-                const Half4 h = load4(res1, a.res1_layout, c, y, x, a.H, a.W, a.Hp, a.Wp);
+                const Half4 h = load4(res1, a.res1_layout, c, y, x, place, live);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + f[v];
             }
             if (res2 != nullptr) {
-                const Half4 h = load4(res2, a.res2_layout, a.res2_coff + c, y, x, a.H, a.W, a.Hp, a.Wp);
+                const Half4 h = load4(res2, a.res2_layout, a.res2_coff + c, y, x, place, live);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) f[v] = half_at(h, v) + (float)round_f16(f[v]);
             }
-            store4(out, a.out_layout, c, y, x, a.H, a.W, a.Hp, a.Wp, pack4(f));
+            store4(out, a.out_layout, c, y, x, place, pack4(f), live);
         }
     }
 }
 
-template <int CB, int TH, int PG>
+template <int KS, int CB, int NH, int N, int TH, int PG>
 hipError_t launch_wide_as(WideConvArgs a, int images, int chunks, hipStream_t stream) {
-    using L = WideConv<CB, TH, PG>;
+    using L = WideConv<KS, CB, NH, N, TH, PG>;
     a.tiles_x = (a.W + kWideTW - 1) / kWideTW;
     a.tiles_image = (a.H + TH - 1) / TH * a.tiles_x;
     a.tiles = images * a.tiles_image;
-    auto kernel = &conv_wide_kernel<CB, TH, PG>;
+    auto kernel = &conv_wide_kernel<KS, CB, NH, N, TH, PG>;
     const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), L::lds);
     if (attr != hipSuccess) return attr;
     hipLaunchKernelGGL(kernel, dim3((unsigned)((a.tiles + 7) / 8 * 8), (unsigned)chunks), dim3(64 * L::NW), L::lds, stream, a);
@@ -575,8 +599,8 @@ namespace {
 template <int CB>
 hipError_t launch_wide_cb(const WideConvArgs& a, int images, int chunks, hipStream_t stream) {
     if constexpr (CB <= 25)
-        if (wide_tiles(a.H, a.W, images, 8) > 256) return launch_wide_as<CB, 8, 2>(a, images, chunks, stream);
-    return launch_wide_as<CB, 4, 2>(a, images, chunks, stream);
+        if (wide_tiles(a.H, a.W, images, 8) > 256) return launch_wide_as<3, CB, 2, 2, 8, 2>(a, images, chunks, stream);
+    return launch_wide_as<3, CB, 2, 2, 4, 2>(a, images, chunks, stream);
 }
 
 }  // namespace
@@ -604,11 +628,10 @@ hipError_t launch_conv3x3_wide(const ConvGeometry& g, const void* x_cb8, const v
     a.out_ts = batch.out;
     a.H = g.h;
     a.W = g.w;
-    a.Hp = g.h + 2 * kPad;
-    a.Wp = g.w + 2 * kPad;
+    a.pad = kPad;
     a.Cout = g.cout;
     a.NBT = g.nbt;
-    a.xin_bytes = (uint32_t)((size_t)g.cb * a.Hp * a.Wp * 16);
+    a.xin_bytes = (uint32_t)((size_t)g.cb * (g.h + 2 * kPad) * (g.w + 2 * kPad) * 16);
     a.wpk_bytes = (uint32_t)conv_packed_bytes(g);
     switch (g.cb) {
         case 8: return launch_wide_cb<8>(a, batch.images, g.chunks, stream);
@@ -618,6 +641,64 @@ hipError_t launch_conv3x3_wide(const ConvGeometry& g, const void* x_cb8, const v
         case 32: return launch_wide_cb<32>(a, batch.images, g.chunks, stream);
         case 40: return launch_wide_cb<40>(a, batch.images, g.chunks, stream);
     }
+    return hipErrorInvalidValue;
+}
+
+namespace {
+
+// The smallest tile whose workgroups fit the 256 CUs at once, else 16 rows, or 8 for the layers
+// with little work per pixel. us per layer (8 -> 32 / 32 -> 64 / 64 -> 32 / 32 -> 16 / 16 -> 2) over 58
+// images, 16x16 at 4 rows 4.8 / 9.7 / 9.9 / 5.3 / 4.6, at 8 rows 5.4 / 10.5 / 11.0 / 6.1 / 5.9; 32x32 at 8
+// rows 6.4 / 19.1 / 18.5 / 8.7 / 6.0, at 16 rows (232 tiles) 7.5 / 15.3 / 16.7 / 9.7 / 7.9; 64x64 at 8 rows
+// 15.8 / 62.1 / 60.9 / 22.0 / 12.1, at 16 rows 16.2 / 48.7 / 45.7 / 21.0 / 13.0 (980 TFLOP/s at 32 -> 64).
+template <int CB, int NH, int N>
+hipError_t launch_convk_as(const WideConvArgs& a, int images, hipStream_t stream) {
+    const auto fits = [&](int th) { return wide_tiles(a.H, a.W, images, th) <= 256; };
+    if (fits(4)) return launch_wide_as<7, CB, NH, N, 4, 2>(a, images, 1, stream);
+    if (N == 1 || CB == 1 || fits(8)) return launch_wide_as<7, CB, NH, N, 8, 4>(a, images, 1, stream);
+    return launch_wide_as<7, CB, NH, N, 16, 4>(a, images, 1, stream);
+}
+
+}  // namespace
+
+// Above two 16-pixel workgroups of convk_kernel per CU, on maps at least a tile wide: SPyNet
+// on one pair (512 of them at 64x64) 151.6 us with convk_kernel, 168.7 with this; on 4 pairs
+// 212.7 against 188.4, on 29 744 against 333.
+bool convk_wide_chosen(const ConvKGeometry& g, int batch, const uint16_t* out, int out_cb8) {
+    const bool layer = (g.cb == 1 && g.nbt == 2) || (g.cb == 4 && g.nbt == 4) || (g.cb == 8 && g.nbt == 2) ||
+                       (g.cb == 4 && g.nbt == 1) || (g.cb == 2 && g.nbt == 1);
+    return g.ks == 7 && g.chunks == 1 && layer && g.w >= kWideTW && (long)batch * g.h * g.w > 512 * 16 &&
+           (!out_cb8 || (g.cout % 4 == 0 && (uintptr_t)out % 8 == 0));
+}
+
+hipError_t launch_convk_wide(const ConvKGeometry& g, int batch, int pad, const void* x_cb8, const void* wpk,
+                             const float* bias, int act, const uint16_t* base, uint16_t* out, int out_cb8,
+                             hipStream_t stream) {
+    WideConvArgs a{};
+    const long padded = (long)(g.h + 2 * pad) * (g.w + 2 * pad) * 8, plane = (long)g.h * g.w;
+    a.xin = x_cb8;
+    a.wpk = wpk;
+    a.bias = bias;
+    a.res2 = base;
+    a.out = out;
+    a.act = act;
+    a.res2_layout = kLayoutNCHW;
+    a.out_layout = out_cb8 ? kLayoutCB8 : kLayoutNCHW;
+    a.H = g.h;
+    a.W = g.w;
+    a.pad = pad;
+    a.Cout = g.cout;
+    a.NBT = g.nbt;
+    a.xin_ts = g.cb * padded;
+    a.res2_ts = g.cout * plane;
+    a.out_ts = out_cb8 ? (g.cout + 7) / 8 * padded : g.cout * plane;
+    a.xin_bytes = (uint32_t)(a.xin_ts * 2);
+    a.wpk_bytes = (uint32_t)convk_packed_bytes(g);
+    if (g.cb == 1 && g.nbt == 2) return launch_convk_as<1, 1, 2>(a, batch, stream);
+    if (g.cb == 4 && g.nbt == 4) return launch_convk_as<4, 2, 2>(a, batch, stream);
+    if (g.cb == 8 && g.nbt == 2) return launch_convk_as<8, 1, 2>(a, batch, stream);
+    if (g.cb == 4 && g.nbt == 1) return launch_convk_as<4, 1, 1>(a, batch, stream);
+    if (g.cb == 2 && g.nbt == 1) return launch_convk_as<2, 1, 1>(a, batch, stream);
     return hipErrorInvalidValue;
 }
 

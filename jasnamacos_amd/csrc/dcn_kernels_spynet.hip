@@ -608,6 +608,8 @@ hipError_t launch_convk(const ConvKGeometry& g, int batch, int pad, const void* 
                         const float* bias, int act, const uint16_t* base, uint16_t* out, int out_cb8,
                         hipStream_t stream) {
     if (pad < g.ks / 2) return hipErrorInvalidValue;
+    if (convk_wide_chosen(g, batch, out, out_cb8))
+        return launch_convk_wide(g, batch, pad, x_cb8, wpk, bias, act, base, out, out_cb8, stream);
     ConvKArgs a{};
     a.xin = x_cb8;
     a.wpk = wpk;
