@@ -521,7 +521,7 @@ dcn_status body_step(dcn_body* body, const void* d_feat_current, const void* d_f
     }
     const long off_ts = cb8_image(body, 8);
     const dcn_conv* c0 = body->offset_conv[0];
-    if (body->tiles == 1) {
+    if (dcn::temporal_conv_chosen(body->h, body->w, body->tiles)) {
         // Second-order flow, the conditions (in LDS only), DCN input, the backbone input's
         // leading [feat_current, prefix...] and the first conv_offset layer in one launch.
         DCN_HIP(ctx, dcn::launch_temporal_conv(c0->g, (const uint16_t*)d_feat_prop, (const uint16_t*)d_feat_current,
@@ -530,14 +530,14 @@ dcn_status body_step(dcn_body* body, const void* d_feat_current, const void* d_f
                                                body->branch, (uint16_t*)d_flow2_out, body->deform_cb8, body->bb_in,
                                                c0->wpk, c0->bias, 0.1f, body->off_a, s, m.warp));
     } else {
-        // Many tiles: the batched conv shares each workgroup's weight fragments over up to
-        // 16 images, which the per-image fused kernel cannot; the temporal preparation
-        // runs as its own kernel into the CB8 conditions.
+        // Many pixels: the conv shares each workgroup's weight fragments over a large tile,
+        // which the fused kernel cannot; the temporal preparation runs as its own kernel
+        // into the CB8 conditions.
         DCN_HIP(ctx, dcn::launch_body_temporal((const uint16_t*)d_feat_prop, (const uint16_t*)d_feat_current,
                                                (const uint16_t*)d_feat_n2, (const uint16_t*)d_flow1,
                                                (const uint16_t*)d_prev_flow, has_second_order ? 1 : 0,
                                                prefix, body->branch, (uint16_t*)d_flow2_out, body->cond_cb8,
-                                               body->deform_cb8, body->bb_in, H, W, s, body->tiles));
+                                               body->deform_cb8, body->bb_in, H, W, s, body->tiles, m.warp));
         dcn::ConvBatch cond_conv;
         cond_conv.images = body->tiles;
         cond_conv.x = cb8_image(body, 25);

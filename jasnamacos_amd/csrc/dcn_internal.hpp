@@ -318,7 +318,7 @@ hipError_t launch_conv3x3_offsets(const ConvGeometry& g, const void* x_cb8, cons
                                   const float* bias, const uint16_t* flow1, const uint16_t* flow2,
                                   uint16_t* offset, uint16_t* mask, hipStream_t stream, int images = 1);
 // One kernel for the body's temporal inputs: second-order flow (NCHW), conditions and
-// the DCN input in CB8, and the backbone input's leading [feat_current, prefix...] in CB8.
+// the DCN input in CB8 (warp_cb8: feat_prop and feat_n2 are CB8 tensors), and the backbone input's leading [feat_current, prefix...] in CB8.
 // Backbone input of a branch's first step: [feat_current, prefix...] and a zero aligned
 // slot, CB8 with 64 * (nprefix + 2) channels.
 hipError_t launch_body_initial(const uint16_t* feat_current, const uint16_t* const* prefix, int nprefix,
@@ -328,7 +328,10 @@ hipError_t launch_body_temporal(const uint16_t* feat_prop, const uint16_t* feat_
                                 const uint16_t* prev_flow, int has_second_order,
                                 const uint16_t* const* prefix, int nprefix, uint16_t* flow2,
                                 uint16_t* cond_cb8, uint16_t* deform_cb8, uint16_t* bb_cb8, int H,
-                                int W, hipStream_t stream, int images = 1);
+                                int W, hipStream_t stream, int images = 1, bool warp_cb8 = false);
+// Whether a step over `tiles` images runs launch_temporal_conv (else launch_body_temporal and
+// launch_conv3x3).
+bool temporal_conv_chosen(int height, int width, int tiles);
 hipError_t launch_second_order_flow(const uint16_t* flow1, const uint16_t* prev, uint16_t* flow2,
                                     int H, int W, int has_second_order, hipStream_t stream);
 hipError_t launch_temporal_assemble(const uint16_t* feat_prop, const uint16_t* feat_current,

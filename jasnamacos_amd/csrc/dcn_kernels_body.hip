@@ -184,15 +184,17 @@ struct BodyImage {
     int nprefix, has_second_order, H, W;
 };
 
-__device__ __forceinline__ BodyImage temporal_image(const BodyTemporalArgs& a0) {
+// warp_cb8: feat_prop and feat_n2 are CB8 tensors.
+__device__ __forceinline__ BodyImage temporal_image(const BodyTemporalArgs& a0, bool warp_cb8 = false) {
     BodyImage a;
     const long z = blockIdx.z;
     const long fs = z * 64 * a0.H * a0.W;  // per-image offset of a feature, then of a flow
     const long ls = z * 2 * a0.H * a0.W;
     const long unit = (long)(a0.H + 2 * kPad) * (a0.W + 2 * kPad) * 8;
-    a.feat_prop = a0.feat_prop + fs;
+    const long ws = warp_cb8 ? z * 8 * unit : fs;
+    a.feat_prop = a0.feat_prop + ws;
     a.feat_current = a0.feat_current + fs;
-    a.feat_n2 = a0.feat_n2 + fs;
+    a.feat_n2 = a0.feat_n2 + ws;
     a.flow1 = a0.flow1 + ls;
     a.prev_flow = a0.prev_flow + ls;
     a.p0 = a0.prefix[0] + fs;
@@ -216,8 +218,9 @@ __device__ __forceinline__ BodyImage temporal_image(const BodyTemporalArgs& a0) 
 // per pixel writes the block's 16 bytes of CB8. The second-order flow of a pixel is
 // recomputed by each thread that needs it (same arithmetic, same bits) and stored by
 // the flow block's thread.
+template <bool WARP_CB8>
 __global__ __launch_bounds__(256) void body_temporal_kernel(BodyTemporalArgs a0) {
-    const BodyImage a = temporal_image(a0);
+    const BodyImage a = temporal_image(a0, WARP_CB8);
     const int plane = a.H * a.W;
     const int p = blockIdx.x * 256 + threadIdx.x;
     if (p >= plane) return;
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(256) void body_temporal_kernel(BodyTemporalArgs a0)
         dst = a.cond;
         dblock = kind;
         uint16_t f2[2];
-        out = condition_block<u32x4>(a.feat_prop, a.feat_current, a.feat_n2, a.flow1, a.prev_flow,
+        out = condition_block<u32x4, WARP_CB8>(a.feat_prop, a.feat_current, a.feat_n2, a.flow1, a.prev_flow,
                                      a.has_second_order, a.H, a.W, kind, y, x, f2);
         if (kind == 24) {
             a.flow2[p] = f2[0];
@@ -241,7 +244,11 @@ __global__ __launch_bounds__(256) void body_temporal_kernel(BodyTemporalArgs a0)
     } else if (kind < 41) {
         dst = a.deform;
         dblock = kind - 25;
-        out = copy8<u32x4>(dblock < 8 ? a.feat_prop + (size_t)dblock * 8 * pl : a.feat_n2 + (size_t)(dblock - 8) * 8 * pl,
+        if constexpr (WARP_CB8)
+            out = reinterpret_cast<const u32x4*>(dblock < 8 ? a.feat_prop : a.feat_n2)
+                [((size_t)(dblock & 7) * (a.H + 2 * kPad) + y + kPad) * (a.W + 2 * kPad) + x + kPad];
+        else
+            out = copy8<u32x4>(dblock < 8 ? a.feat_prop + (size_t)dblock * 8 * pl : a.feat_n2 + (size_t)(dblock - 8) * 8 * pl,
                            pl, p);
     } else {
         dst = a.bb;
@@ -308,7 +315,7 @@ hipError_t launch_body_temporal(const uint16_t* feat_prop, const uint16_t* feat_
                                 const uint16_t* prev_flow, int has_second_order,
                                 const uint16_t* const* prefix, int nprefix, uint16_t* flow2,
                                 uint16_t* cond_cb8, uint16_t* deform_cb8, uint16_t* bb_cb8, int H,
-                                int W, hipStream_t stream, int images) {
+                                int W, hipStream_t stream, int images, bool warp_cb8) {
     if (nprefix < 0 || nprefix > 3 || images < 1) return hipErrorInvalidValue;
     BodyTemporalArgs a{};
     a.feat_prop = feat_prop;
@@ -326,7 +333,7 @@ hipError_t launch_body_temporal(const uint16_t* feat_prop, const uint16_t* feat_
     a.deform = deform_cb8;
     a.bb = bb_cb8;
     const dim3 grid(blocks_for((long)H * W), (unsigned)(41 + 8 * (1 + nprefix)), (unsigned)images);
-    hipLaunchKernelGGL(body_temporal_kernel, grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(warp_cb8 ? body_temporal_kernel<true> : body_temporal_kernel<false>, grid, dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

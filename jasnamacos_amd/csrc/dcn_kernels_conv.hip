@@ -1308,6 +1308,13 @@ hipError_t launch_conv3x3_offsets(const ConvGeometry& g, const void* x_cb8, cons
     return hipGetLastError();
 }
 
+// One image of at most 256 tiles of 2 x 8 pixels, one workgroup per CU; beyond that each round
+// of workgroups samples 2.5 times the pixels it outputs and fetches all weights again (150x150:
+// 50 us, against 14 + 10 for the two kernels).
+bool temporal_conv_chosen(int height, int width, int tiles) {
+    return tiles == 1 && (long)((height + kTcTH - 1) / kTcTH) * ((width + kTcTW - 1) / kTcTW) <= 256;
+}
+
 hipError_t launch_temporal_conv(const ConvGeometry& g, const uint16_t* feat_prop, const uint16_t* feat_current,
                                 const uint16_t* feat_n2, const uint16_t* flow1, const uint16_t* prev_flow,
                                 int has_second_order, const uint16_t* const* prefix, int nprefix,

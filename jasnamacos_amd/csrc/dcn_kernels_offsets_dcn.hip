@@ -6,16 +6,16 @@
 // (the DCN samples straight from the conv's output, with no HBM round trip), and a frame
 // saves one launch and one kernel's load/reduce latency chain.
 //
-// Workgroup: 12 waves on one 16-pixel tile of up to four images (grid z = image group).
-//  * Phase A, the offsets conv: the tile's A fragments (18 K-steps of 64 lanes per image)
+// Workgroup: 12 waves on up to four consecutive 16-pixel tiles of an image.
+//  * Phase A, the offsets conv: the tiles' A fragments (18 K-steps of 64 lanes each)
 //    are staged in LDS once; wave w owns 16-channel column blocks w, w + 12 (and w + 24 for
 //    w < 3) of the 27 and runs every K-step for them, streaming its weight fragments and
-//    applying each to every image of the group. The K range is
+//    applying each to every tile of the group. The K range is
 //    summed in conv_offsets_kernel's order: chains over the eight ranges
 //    [r * 18 / 8, (r + 1) * 18 / 8) from zero, added to a zero sum in range order, so each
 //    raw value, and each offset and mask after prepare_dcn_offsets_fp16
 //    (MetalShader.swift:815-839), is the same bits as conv_offsets_kernel's.
-//  * Phase B, the DCN, image by image with the weight fragments held in registers:
+//  * Phase B, the DCN, tile by tile with the weight fragments held in registers:
 //    narrow_kernel<4, 12, 3> with the offsets and masks read from LDS (same K split, blend
 //    and summation order): the aligned feature is the same bits as the two-kernel path.
 #include <hip/hip_runtime.h>
@@ -44,15 +44,15 @@ constexpr int kDcnKsteps = 36;                 // 128 channels x 9 taps / 32
 constexpr int kDcnNb = 4;                      // 64 output channels
 constexpr int kDcnPerWave = kDcnKsteps / kOdWaves;
 
-constexpr size_t kStageBytes = (size_t)kOffKsteps * 64 * 16;       // A fragments of an image
-constexpr size_t kOffsBytes = (size_t)kOffChannels * 16 * 2;        // [432][16] FP16 per image
+constexpr size_t kStageBytes = (size_t)kOffKsteps * 64 * 16;       // A fragments of a tile
+constexpr size_t kOffsBytes = (size_t)kOffChannels * 16 * 2;        // [432][16] FP16 per tile
 constexpr int kOdRedStride = 68;  // partial-sum rows of 64 lanes, padded: conflict-free channel-fastest reads
 constexpr size_t kRedBytes = (size_t)kOdWaves * kDcnNb * 4 * kOdRedStride * 4;
-constexpr size_t kFlowBytes = 2 * 2 * 16 * 2;                      // [flow][channel][16] FP16 per image
-// From three images on, the DCN's partial sums reuse the A-fragment stage (dead by then).
-__host__ __device__ constexpr bool od_red_in_stage(int images) { return images * kStageBytes >= kRedBytes; }
-__host__ __device__ constexpr size_t od_lds_bytes(int images) {
-    return (size_t)images * (kStageBytes + kOffsBytes + kFlowBytes) + (od_red_in_stage(images) ? 0 : kRedBytes);
+constexpr size_t kFlowBytes = 2 * 2 * 16 * 2;                      // [flow][channel][16] FP16 per tile
+// From three tiles on, the DCN's partial sums reuse the A-fragment stage (dead by then).
+__host__ __device__ constexpr bool od_red_in_stage(int tiles) { return tiles * kStageBytes >= kRedBytes; }
+__host__ __device__ constexpr size_t od_lds_bytes(int tiles) {
+    return (size_t)tiles * (kStageBytes + kOffsBytes + kFlowBytes) + (od_red_in_stage(tiles) ? 0 : kRedBytes);
 }
 
 // Bit s set when K-step s ends one of the eight K ranges of conv_offsets_kernel.
@@ -74,13 +74,15 @@ struct OffsetsDcnArgs {
     const float* bdcn;      // [64]
     uint16_t* out;          // CB8 backbone input, per image out_ts
     uint32_t xoff_bytes, woff_bytes, xin_bytes, wdcn_bytes;
-    int H, W, Hp, Wp, nbt, tiles, out_coff, out_cblk, images;
+    int H, W, Hp, Wp, nbt, tiles, groups, out_coff, out_cblk;  // tiles and workgroups of one image
+    uint32_t all_groups;
+    uint64_t magic_groups;  // ceil(2^40 / groups): exact for fewer than 2^20 workgroups
     long xoff_ts, flow_ts, xin_ts, out_ts;
 };
 
-// Workgroup (tile, zg) runs images zg * Z .. zg * Z + Z - 1 (fewer in the last group):
-// phase A for all of them at once (each weight fragment applied to every image's A
-// fragment), then phase B image by image with the DCN weights held in registers.
+// Workgroup g runs tiles g * Z .. g * Z + Z - 1 (fewer in the last one): phase A for all of them
+// at once (each weight fragment applied to every tile's A fragment), then phase B tile by
+// tile with the DCN weights held in registers.
 template <int SAMPLER, int Z>
 __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -95,16 +97,21 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
     const int wave = tid >> 6;
     const int quarter = lane >> 4;
 
-    const int per_xcd = (a.tiles + 7) / 8;
-    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (tile >= a.tiles) return;  // whole workgroup, before any barrier
-    const long z0 = (long)blockIdx.z * Z;
-    const int nimg = (int)min((long)Z, (long)a.images - z0);  // uniform, >= 1
+    // An XCD runs a band of the workgroups of all images; only the grid's last row of eight has
+    // empty ones. (With empty ones in every image's last row the dispatcher, which gives each
+    // shader engine its turn whatever the workgroup does, put two on some CUs with others
+    // idle: 5 images of 50 workgroups 42 us against 21.)
+    const uint32_t per_xcd = (a.all_groups + 7) / 8;
+    const uint32_t wg = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (wg >= a.all_groups) return;  // whole workgroup, before any barrier
+    const long z = (long)(((uint64_t)wg * a.magic_groups) >> 40);  // wg / a.groups: image
+    const int tile0 = (int)(wg - (uint32_t)z * (uint32_t)a.groups) * Z;
+    const int nt = min(Z, a.tiles - tile0);  // uniform, >= 1
     const int M = a.H * a.W;
     const __amdgpu_buffer_rsrc_t wor = make_rsrc(a.woff, a.woff_bytes);
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.wdcn, a.wdcn_bytes);
 
-    // ---- phase A: the offsets conv on this tile ----------------------------------------
+    // ---- phase A: the offsets conv on the tiles ---------------------------------------
     // Column blocks of this wave.
     const int nblocks = wave < kOffBlocks - 2 * kOdWaves ? 3 : 2;
     // The DCN epilogue's biases (output channel idx / 16 of items idx = tid, tid + 768) and
@@ -139,30 +146,29 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
         for (int s = 0; s < kOffRing; ++s) load_b(s, s, Two{});
     }
 
-    // The tile's flows (both flows, both channels, 16 pixels per image; a clamped pixel,
+    // The tiles' flows (both flows, both channels, 16 pixels per tile; a clamped pixel,
     // zeroed when written), requested before the A fragments.
-    const int px_flow = tile * 16 + (tid & 15);
+    int px_flow = 0;
     uint16_t flow_v = 0;
-    if (tid < nimg * 64) {  // whole waves
-        const int img = tid >> 6;
+    if (tid < nt * 64) {  // whole waves
+        px_flow = (tile0 + wave) * 16 + (tid & 15);
         const int f = (tid >> 5) & 1;
         const int c = (tid >> 4) & 1;
-        const uint16_t* flow = (f == 0 ? a.flow1 : a.flow2) + (z0 + img) * a.flow_ts;
+        const uint16_t* flow = (f == 0 ? a.flow1 : a.flow2) + z * a.flow_ts;
         flow_v = flow[c * (size_t)M + min(px_flow, M - 1)];
     }
     // A fragment of K-step s, lane l: pixel l % 16 (clamped into the image), K-block
     // 4 s + l / 16 = tap * 8 + cb, as conv_offsets_kernel loads it; copied straight into
     // LDS (buffer_load ... lds: lane l's 16 bytes land at the wave's base + 16 l), so no
     // load waits for the one before it.
-    for (int u0 = __builtin_amdgcn_readfirstlane(wave) * 64; u0 < nimg * kOffKsteps * 64; u0 += kOdThreads) {
+    const __amdgpu_buffer_rsrc_t xor_ = make_rsrc(static_cast<const uint16_t*>(a.xoff) + z * a.xoff_ts, a.xoff_bytes);
+    for (int u0 = __builtin_amdgcn_readfirstlane(wave) * 64; u0 < nt * kOffKsteps * 64; u0 += kOdThreads) {
         const int u = u0 + lane;
-        const int img = u0 / (kOffKsteps * 64);  // wave-uniform: 64 divides an image's units
-        const int r = u - img * (kOffKsteps * 64);
+        const int t = u0 / (kOffKsteps * 64);  // wave-uniform: 64 divides a tile's units
+        const int r = u - t * (kOffKsteps * 64);
         const int s = r >> 6;
         const int l = r & 63;
-        const __amdgpu_buffer_rsrc_t xor_ =
-            make_rsrc(static_cast<const uint16_t*>(a.xoff) + (z0 + img) * a.xoff_ts, a.xoff_bytes);
-        const int pc = min(tile * 16 + (l & 15), M - 1);
+        const int pc = min((tile0 + t) * 16 + (l & 15), M - 1);
         const int y = pc / a.W;
         const uint32_t base = (uint32_t)(y + kPad - 1) * a.Wp + (pc - y * a.W) + kPad - 1;
         const int kb = 4 * s + (l >> 4);
@@ -170,13 +176,13 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
         const int cb = kb & 7;
         const int ky = (tap * 11) >> 5;  // tap / 3 for tap < 9
         const int kx = tap - ky * 3;
-        if (u < nimg * kOffKsteps * 64)
+        if (u < nt * kOffKsteps * 64)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 xor_, (__attribute__((address_space(3))) void*)(stage + u0),
                 16, (int)((base + (uint32_t)(cb * a.Hp + ky) * a.Wp + kx) * 16u), 0, 0, 0);
     }
     __builtin_amdgcn_s_waitcnt(0);  // this wave's copies (the compiler does not track them)
-    if (tid < nimg * 64) flows[tid] = px_flow < M ? flow_v : (uint16_t)0;
+    if (tid < nt * 64) flows[tid] = px_flow < M ? flow_v : (uint16_t)0;
     __syncthreads();  // A fragments staged, flows in LDS
 
     f32x4 acc[Z][3], sum[Z][3];
@@ -197,7 +203,7 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
                 const int s = sg + slot;
 #pragma unroll
                 for (int i = 0; i < Z; ++i) {
-                    if (i >= nimg) continue;
+                    if (i >= nt) continue;
                     const h8 A = __builtin_bit_cast(h8, stage[(i * kOffKsteps + s) * 64 + lane]);
 #pragma unroll
                     for (int j = 0; j < NBL; ++j)
@@ -217,9 +223,9 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
                 }
             }
         };
-        // One image: unrolled (a rolled loop's header merges the wait state of its back
+        // One tile: unrolled (a rolled loop's header merges the wait state of its back
         // edge and waits for every slot), a scheduling barrier per K-step keeping later
-        // loads where they are. Batches stay rolled (unrolled, their accumulators spill).
+        // loads where they are. More tiles stay rolled (unrolled, their accumulators spill).
         if constexpr (Z == 1) {
 #pragma unroll
             for (int sg = 0; sg < kOffKsteps; sg += kOffRing) group(sg);
@@ -251,7 +257,7 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
         const float bias = boffv[j];
 #pragma unroll
         for (int i = 0; i < Z; ++i) {
-            if (i >= nimg) continue;
+            if (i >= nt) continue;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int px = 4 * quarter + v;
@@ -274,20 +280,19 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
     __syncthreads();  // offsets and masks of the tile complete
 
     // ---- phase B: the DCN (narrow_kernel<4, 12, 3> with offsets from LDS) ---------------
-    const int p = tile * 16 + (lane & 15);
-    const bool pvalid = p < M;
-    const int sp = pvalid ? p : M - 1;
-    const int oy = sp / a.W;
-    const int ox = sp - oy * a.W;
-    const int base_y = oy - 1;  // stride 1, pad 1
-    const int base_x = ox - 1;
     const uint32_t xinb = (uint32_t)kPad * a.Wp + kPad;  // 16-byte units, border shift
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(static_cast<const uint16_t*>(a.xin) + z * a.xin_ts, a.xin_bytes);
+    uint16_t* out = a.out + z * a.out_ts;
 
-    for (int img = 0; img < nimg; ++img) {
-        const long z = z0 + img;
-        const __amdgpu_buffer_rsrc_t xr =
-            make_rsrc(static_cast<const uint16_t*>(a.xin) + z * a.xin_ts, a.xin_bytes);
-        const uint16_t* io = offs + img * kOffChannels * 16;
+    for (int t = 0; t < nt; ++t) {
+        const int p = (tile0 + t) * 16 + (lane & 15);
+        const bool pvalid = p < M;
+        const int sp = pvalid ? p : M - 1;
+        const int oy = sp / a.W;
+        const int ox = sp - oy * a.W;
+        const int base_y = oy - 1;  // stride 1, pad 1
+        const int base_x = ox - 1;
+        const uint16_t* io = offs + t * kOffChannels * 16;
         u32x4 q[kDcnPerWave][4];
         float ly[kDcnPerWave], lx[kDcnPerWave], m[kDcnPerWave];
 #pragma unroll
@@ -328,14 +333,13 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
             for (int nb = 0; nb < kDcnNb; ++nb)
                 dacc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, Bf[i][nb], dacc[nb], 0, 0, 0);
         }
-        if (img > 0) __syncthreads();  // the previous image's sums were read
+        if (t > 0) __syncthreads();  // the previous tile's sums were read
 #pragma unroll
         for (int nb = 0; nb < kDcnNb; ++nb)
 #pragma unroll
             for (int v = 0; v < 4; ++v) red[((wave * kDcnNb + nb) * 4 + v) * kOdRedStride + lane] = dacc[nb][v];
         __syncthreads();
 
-        uint16_t* out = a.out + z * a.out_ts;
 #pragma unroll
         for (int k = 0; k < kDcnIters; ++k) {
             const int idx = tid + k * kOdThreads;
@@ -362,11 +366,16 @@ __global__ __launch_bounds__(kOdThreads) void offsets_dcn_kernel(OffsetsDcnArgs 
 }
 
 template <int Z>
-hipError_t launch_od_t(const OffsetsDcnArgs& a, hipStream_t stream) {
+hipError_t launch_od_t(OffsetsDcnArgs a, int images, hipStream_t stream) {
+    a.groups = (a.tiles + Z - 1) / Z;
+    const long all = (long)a.groups * images;
+    if (all >= 1 << 20) return hipErrorInvalidValue;
+    a.all_groups = (uint32_t)all;
+    a.magic_groups = (((uint64_t)1 << 40) + a.groups - 1) / a.groups;
     auto kernel = &offsets_dcn_kernel<kSamplerFast, Z>;
     const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), od_lds_bytes(Z));
     if (attr != hipSuccess) return attr;
-    const dim3 grid((unsigned)((a.tiles + 7) / 8 * 8), 1, (unsigned)((a.images + Z - 1) / Z));
+    const dim3 grid((unsigned)((all + 7) / 8 * 8));
     hipLaunchKernelGGL(kernel, grid, dim3(kOdThreads), od_lds_bytes(Z), stream, a);
     return hipGetLastError();
 }
@@ -408,14 +417,13 @@ hipError_t launch_offsets_dcn(const ConvGeometry& goff, const void* xoff_cb8, co
     a.xin_bytes = (uint32_t)(a.xin_ts * 2);
     a.woff_bytes = (uint32_t)conv_packed_bytes(goff);
     a.wdcn_bytes = (uint32_t)wdcn_bytes;
-    a.images = images;
-    // Images per workgroup: up to four (LDS 130 KB, the DCN's sums in the dead stage),
-    // measured for a body step over 16 tiles: 621 us (one), 580 (two), 574 (three), 565
-    // (four); over 64 tiles 2478, 2294, 2258, 2230 us.
-    if (images >= 4) return launch_od_t<4>(a, stream);
-    if (images >= 3) return launch_od_t<3>(a, stream);
-    if (images == 2) return launch_od_t<2>(a, stream);
-    return launch_od_t<1>(a, stream);
+    // As many tiles per workgroup as leave one workgroup per CU, up to four (LDS 130 KB, the
+    // DCN's sums in the dead stage).
+    const long all = (long)images * a.tiles;
+    if (all > 768) return launch_od_t<4>(a, images, stream);
+    if (all > 512) return launch_od_t<3>(a, images, stream);
+    if (all > 256) return launch_od_t<2>(a, images, stream);
+    return launch_od_t<1>(a, images, stream);
 }
 
 }  // namespace dcn
