@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 
 #include "dcn_device.hpp"
 #include "dcn_internal.hpp"
@@ -438,25 +439,36 @@ __global__ __launch_bounds__(64 * NW) void narrow_images_kernel(NarrowArgs a, in
     }
 }
 
-// Images per workgroup of the batched narrow kernel: up to 16, balanced over the
-// workgroups of a tile. Measured for a body step over 16 tiles (images per workgroup ->
-// us per step): 2 -> 642, 4 -> 632, 8 -> 628, 16 -> 627 (654 with one image per
-// workgroup of narrow_kernel).
-static int narrow_images_per_group(int images) {
-    constexpr int kMax = 16;
-    const int groups = (images + kMax - 1) / kMax;
-    return (images + groups - 1) / groups;
+// Images per workgroup of the batched narrow kernel, `tiles` 16-pixel tiles per image: up to
+// 16, with the fewest rounds of 256 workgroups (one per CU) times the time of one, which is
+// about that of its images plus one more (4 maps of 64x64, 256 workgroups of 4: 33 us; 7: 51 us).
+// Many small maps take fewer images each. Against 16 whatever the map: 16 maps of 16x16 (16
+// workgroups, now 256) 83.6 -> 10.0 us, 16 of 40x45 107 -> 59, 9 of 24x31 61 -> 21, 12 of 48x48
+// 81 -> 63.
+// Over many rounds the choice hardly matters (a body step over 16 tiles of 64x64 at 2 / 4 / 8 /
+// 16: 642 / 632 / 628 / 627 us).
+static int narrow_images_per_group(int images, int tiles) {
+    int best = 1;
+    long best_cost = LONG_MAX;
+    for (int zpw = std::min(images, 16); zpw >= 1; --zpw) {
+        const long groups = (images + zpw - 1) / zpw;
+        const long cost = (groups * tiles + 255) / 256 * (zpw + 1);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = (int)((images + groups - 1) / groups);
+        }
+    }
+    return best;
 }
 
 template <int NB, int NW, int SAMPLER>
-hipError_t launch_narrow_images_t(NarrowArgs a, int images, hipStream_t stream) {
+hipError_t launch_narrow_images_t(NarrowArgs a, int images, int zpw, hipStream_t stream) {
     constexpr int KMAX = 3;
     const size_t lds = (size_t)NW * NB * 4 * 65 * sizeof(float);
     auto kernel = &narrow_images_kernel<NB, NW, KMAX, SAMPLER>;
     const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)lds);
     if (attr != hipSuccess) return attr;
     a.tiles = (a.HWo + 15) / 16;  // per image
-    const int zpw = narrow_images_per_group(images);
     const dim3 grid((unsigned)((a.tiles + 7) / 8 * 8), 1, (unsigned)((images + zpw - 1) / zpw));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, stream, a, images, zpw);
     return hipGetLastError();
@@ -556,11 +568,12 @@ hipError_t launch_narrow_f16(const KShape& s, const FusedGeometry& g, const Fuse
     // Batches of images whose K range fits three K-steps per wave (the body's 128 -> 64
     // DCN over many tiles): weights stay in registers across the images of a workgroup.
     // From four images on (C3's tiles at batch 2: 19.5 us against 18.6 us for
-    // narrow_kernel; at batch 4: 33.0 against 33.7 us).
+    // narrow_kernel; at batch 4: 33.0 against 33.7 us), where a workgroup gets two or more.
     if (cfg.sampler == kSamplerBf16) return launch_narrow_s<kSamplerBf16>(a, g.nb * 2, cfg.ks, stream);
-    if (s.B >= 4 && g.nb * 2 == 4 && cfg.ks == 12 && (a.ksteps + 11) / 12 <= 3)
-        return cfg.sampler == kSamplerExact ? launch_narrow_images_t<4, 12, kSamplerExact>(a, s.B, stream)
-                                            : launch_narrow_images_t<4, 12, kSamplerFast>(a, s.B, stream);
+    const int zpw = narrow_images_per_group(s.B, (a.HWo + 15) / 16);
+    if (s.B >= 4 && zpw >= 2 && g.nb * 2 == 4 && cfg.ks == 12 && (a.ksteps + 11) / 12 <= 3)
+        return cfg.sampler == kSamplerExact ? launch_narrow_images_t<4, 12, kSamplerExact>(a, s.B, zpw, stream)
+                                            : launch_narrow_images_t<4, 12, kSamplerFast>(a, s.B, zpw, stream);
     if (cfg.sampler == kSamplerExact) return launch_narrow_s<kSamplerExact>(a, g.nb * 2, cfg.ks, stream);
     return launch_narrow_s<kSamplerFast>(a, g.nb * 2, cfg.ks, stream);
 }
