@@ -66,7 +66,7 @@ WORKLOADS = {
 }
 
 
-KERNEL_NAMES = {0: "direct_shared_f32_kernel", 1: "fused_kernel", 2: "staged_kernel", 3: "window_kernel", 4: "window_kernel",
+KERNEL_NAMES = {0: "shared_kernel", 1: "fused_kernel", 2: "staged_kernel", 3: "window_kernel", 4: "window_kernel",
                 5: "narrow_kernel", 6: "window_async_kernel", 7: "tile_kernel"}
 
 
