@@ -131,6 +131,15 @@ hipError_t launch_tile_f16(const KShape& s, const FusedGeometry& g, const FusedC
                            hipStream_t stream, unsigned long long* clock = nullptr);
 size_t tile_grid(const KShape& s, const FusedConfig& cfg);  // workgroups of a tile launch
 
+// Plain-weight forwards, shared samples (dcn_kernels_direct.hip): input channels of a stage,
+// and where stage `st`'s elements start in an output channel's run of weights. `whole` is the
+// run's number of whole stages, one or more; past the last one its start again, so that a
+// load one stage ahead stays in the run.
+constexpr int kSharedCh = 16;
+constexpr int shared_stage_start(int st, int whole, int taps) {
+    return (st < whole ? st : whole - 1) * kSharedCh * taps;
+}
+
 // ---- launchers (return hipSuccess or the launch error) ---------------------------
 hipError_t launch_direct_f32(const KShape& s, const float* in, const float* off,
                              const float* mask, const float* w, const float* b, float* out,

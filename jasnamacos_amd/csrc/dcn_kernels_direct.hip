@@ -143,7 +143,10 @@ hipError_t launch_direct(const KShape& s, const T* in, const T* off, const T* ma
 // OCL * (l / 16) + e, the 16 lanes of a row share their channels, and each keeps one weight of
 // every 16 consecutive (ic, tap) in a register that the multiply reads through a DPP row
 // broadcast (4.2 clocks against 3.1 for a plain multiply, measured). Weights go from memory
-// to registers, one stage ahead. 34.9 -> 28.0 us FP32; FP16 2x128x45x61 -> 64, which ran
+// to registers, one whole stage ahead; the stage is in the load's scalar offset, which the
+// buffer's range check may leave out, so these loads stay inside a channel's run by
+// themselves (shared_stage_start), and the partial stage's have their address in the vector
+// offset. 34.9 -> 28.0 us FP32; FP16 2x128x45x61 -> 64, which ran
 // direct_kernel, 1584 -> 48.7 us (343 workgroups on 256 CUs; 45x61 alone 25.5 us). The corner
 // gathers come next: a pixel's samples are a cache line per channel and corner row, so the
 // two columns of a row are one load (four single loads: 38.6 us against 28.0).
@@ -155,7 +158,6 @@ hipError_t launch_direct(const KShape& s, const T* in, const T* off, const T* ma
 // also wait for the gathers. A sampling item is one (pixel, tap) of CPI channels that
 // share an offset group: position and corner weights once, CPI x 4 corner loads.
 constexpr int kSharedPix = 16;
-constexpr int kSharedCh = 16;
 
 template <typename T>
 struct SharedArgs {
@@ -357,8 +359,9 @@ __global__ __launch_bounds__(64 * (NW + SharedLayout<KA, CPI>::SW)) void shared_
     }
 
     // Chain waves. This row's weights: chunk c of a stage is lane p's element 16 c + p of the
-    // stage's (ic, tap) run. Channels past the group's load its last one, elements past a
-    // channel's run the next one's or zero: nothing uses them.
+    // stage's (ic, tap) run. Channels past the group's load its last one. Elements past a
+    // channel's run, in the partial stage, are the next one's or, past the tensor, zero
+    // (the buffer's range check): nothing uses them.
     const int oc0 = (blockIdx.y - group * a.oc_tiles) * (4 * NW * OCL) + (threadIdx.x >> 4) * OCL;  // in the group
     const __amdgpu_buffer_rsrc_t wr = dev::make_rsrc(a.weight, a.weight_bytes);
     uint32_t wbase[OCL];
@@ -369,16 +372,21 @@ __global__ __launch_bounds__(64 * (NW + SharedLayout<KA, CPI>::SW)) void shared_
         wbase[e] = (uint32_t)oc * (uint32_t)(a.cpg * KA) + p;
         acc[e] = widen(a.bias[oc]);
     }
+    const int full = a.cpg / kSharedCh;  // whole stages
+    auto load_weights = [&](int st, int c) {
+        const uint32_t soff = (uint32_t)(shared_stage_start(st, full, KA) + 16 * c) * (uint32_t)sizeof(T);
+#pragma unroll
+        for (int e = 0; e < OCL; ++e) w[c][e] = load_widened<T>(wr, wbase[e], soff);
+    };
     auto load_run = [&](int j0, float (&v)[OCL]) {
 #pragma unroll
-        for (int e = 0; e < OCL; ++e) v[e] = load_widened<T>(wr, wbase[e], (uint32_t)j0 * (uint32_t)sizeof(T));
+        for (int e = 0; e < OCL; ++e) v[e] = load_widened<T>(wr, wbase[e] + (uint32_t)j0);
     };
-    auto load_weights = [&](int st, int c) { load_run(st * L::J + 16 * c, w[c]); };
     auto row4 = [&](int nb, int j) { return *reinterpret_cast<const float4*>(&sm[nb][p][j]); };
+    if (full > 0)
 #pragma unroll
-    for (int c = 0; c < KA; ++c) load_weights(0, c);
+        for (int c = 0; c < KA; ++c) load_weights(0, c);
     __syncthreads();
-    const int full = a.cpg / kSharedCh;  // whole stages
 #pragma unroll 1
     for (int st = 0; st < full; ++st) {
         const int nb = st & 1;
@@ -399,7 +407,7 @@ __global__ __launch_bounds__(64 * (NW + SharedLayout<KA, CPI>::SW)) void shared_
         // The last, partial stage: its weights again, a chunk ahead.
         const int nb = full & 1;
         const int count = (a.cpg - full * kSharedCh) * KA;
-        load_weights(full, 0);
+        load_run(full * L::J, w[0]);
 #pragma unroll 1
         for (int c = 0; 16 * c < count; ++c) {
             float wt[OCL];

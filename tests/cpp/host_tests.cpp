@@ -13,6 +13,8 @@
 // Usage: host_tests cpu | gpu   (exit status 0 when every test of the group passes)
 #include "dcn/deform_conv.hpp"
 
+#include "dcn_internal.hpp"  // the rules that choose kernels: host code, no device
+
 #include <unistd.h>
 
 #include <cmath>
@@ -446,6 +448,24 @@ TEST(gpu, bicubicQuarterKeepsAConstantImageConstant) {
     const auto out = runner.bicubicQuarter(3, 256, 256, in);
     EXPECT(out.size() == (size_t)3 * 64 * 64);
     for (uint16_t v : out) EXPECT(v == dcn_f32_to_f16(0.375f));
+}
+
+// ---- rules of the kernels' launches (host code, no device) ----------------------------
+
+// The shared-sample kernel's chain waves load stage 0's weights, and during stage st those of
+// stage st + 1, with no range check on the stage's part of the address: every lane of every
+// chunk stays inside its output channel's run.
+TEST(cpu, sharedKernelWeightLoadsStayInTheRun) {
+    for (const int taps : {1, 2, 3, 4, 6, 9})
+        for (int channels = dcn::kSharedCh; channels <= 5 * dcn::kSharedCh; ++channels) {
+            const int run = channels * taps, whole = channels / dcn::kSharedCh;
+            for (int st = 0; st <= whole; ++st) {
+                const int start = dcn::shared_stage_start(st, whole, taps);
+                EXPECT(start >= 0);
+                if (st < whole) EXPECT(start == st * dcn::kSharedCh * taps);
+                for (int chunk = 0; chunk < taps; ++chunk) EXPECT(start + 16 * chunk + 15 < run);
+            }
+        }
 }
 
 }  // namespace

@@ -22,6 +22,9 @@ SHAPES = [
     ((1, 16, 65, 66, 70, 65, 66, 3, 3, 1, 1, 1, 1, 1, 1, 1, 2), 12.0),  # over 256 pixel tiles, 64 + 6 channels
     ((1, 16, 50, 60, 24, 50, 60, 3, 3, 1, 1, 1, 1, 2, 2, 1, 4), 12.0),  # 188 pixel tiles, 24 channels, dilation
     ((1, 32, 70, 64, 24, 70, 64, 3, 3, 1, 1, 1, 1, 1, 1, 2, 2), 12.0),  # over 256 workgroups of 12 channels
+    ((1, 4, 9, 10, 1, 9, 10, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1), 3.0),       # 36 weights in all: less than a stage
+    ((1, 16, 9, 10, 1, 9, 10, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1), 3.0),      # one output channel, one whole stage
+    ((1, 33, 9, 10, 2, 9, 10, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1), 3.0),      # two whole stages and one channel
 ]
 
 
