@@ -139,6 +139,9 @@ constexpr int kSharedCh = 16;
 constexpr int shared_stage_start(int st, int whole, int taps) {
     return (st < whole ? st : whole - 1) * kSharedCh * taps;
 }
+// Whether a plain-weight forward over `element`-byte values runs the shared-sample kernel
+// (else one thread per output).
+bool shared_forward_chosen(const KShape& s, size_t element);
 
 // ---- launchers (return hipSuccess or the launch error) ---------------------------
 hipError_t launch_direct_f32(const KShape& s, const float* in, const float* off,

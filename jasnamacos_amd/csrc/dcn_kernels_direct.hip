@@ -170,12 +170,16 @@ struct SharedArgs {
     uint32_t off_bytes, mask_bytes, weight_bytes;
 };
 
+constexpr int shared_sampling_waves(int ka, int cpi) {
+    const int items = kSharedPix * ka * (kSharedCh / cpi);
+    return items >= 512 ? 8 : (items + 63) / 64;
+}
 template <int KA, int CPI>
 struct SharedLayout {
     static constexpr int J = kSharedCh * KA;
     static constexpr int JP = J + 4;  // padded row (floats): 16-byte aligned rows, odd in 16-byte units
     static constexpr int ITEMS = kSharedPix * KA * (kSharedCh / CPI);
-    static constexpr int SW = ITEMS >= 512 ? 8 : (ITEMS + 63) / 64;  // sampling waves
+    static constexpr int SW = shared_sampling_waves(KA, CPI);
     static constexpr int PER = (ITEMS + 64 * SW - 1) / (64 * SW);    // items per sampling lane
 };
 
@@ -454,54 +458,81 @@ hipError_t launch_shared_as(SharedArgs<T> a, hipStream_t stream) {
 // 32x32 pixels (64 pixel tiles) 17.0 / 18.4 / 22.6, 45x61 (172) 41.9 / 34.9 / 25.5, 64x64 (256)
 // 69.5 / 34.3 / 28.0. Up to 16 channels on more than 256 workgroups take two chain waves of
 // two channels per lane: 2x60x60, 4 groups of 24 -> 10, 30.3 -> 26.5 us.
+struct SharedSplit {
+    int nw, ocl;  // chain waves, output channels per lane
+};
+SharedSplit shared_split(long tiles, int opg) {
+    const auto fits = [&](int oc) { return tiles * ((opg + oc - 1) / oc) <= 256; };
+    if (fits(16)) return {4, 1};
+    if (opg <= 16) return {2, 2};
+    if (opg <= 32 || fits(32)) return {4, 2};
+    return {8, 2};
+}
+// Pixel tiles over all groups.
+long shared_tiles(const KShape& s) {
+    return ((long)s.B * s.Ho * s.Wo + kSharedPix - 1) / kSharedPix * s.groups;
+}
+// Input channels of a sampling item.
+int shared_item_channels(const KShape& s) {
+    if (s.KH * s.KW != 9) return 1;
+    const int both = (s.Cin / s.groups) | (s.Cin / s.og);
+    return both % 8 == 0 ? 8 : both % 4 == 0 ? 4 : 1;
+}
+
 template <typename T, int KA, int CPI>
 hipError_t launch_shared_ka(const SharedArgs<T>& a, hipStream_t stream) {
-    const long tiles = (a.pixels + kSharedPix - 1) / kSharedPix * a.s.groups;
-    const auto fits = [&](int oc) { return tiles * ((a.opg + oc - 1) / oc) <= 256; };
-    if (fits(16)) return launch_shared_as<T, KA, 4, 1, CPI>(a, stream);
-    if (a.opg <= 16) return launch_shared_as<T, KA, 2, 2, CPI>(a, stream);
-    if (a.opg <= 32 || fits(32)) return launch_shared_as<T, KA, 4, 2, CPI>(a, stream);
-    return launch_shared_as<T, KA, 8, 2, CPI>(a, stream);
+    const SharedSplit p = shared_split(shared_tiles(a.s), a.opg);
+    if (p.nw == 2) return launch_shared_as<T, KA, 2, 2, CPI>(a, stream);
+    if (p.nw == 8) return launch_shared_as<T, KA, 8, 2, CPI>(a, stream);
+    return p.ocl == 1 ? launch_shared_as<T, KA, 4, 1, CPI>(a, stream) : launch_shared_as<T, KA, 4, 2, CPI>(a, stream);
 }
 
 template <typename T>
 hipError_t launch_forward(const KShape& s, const T* in, const T* off, const T* mask, const T* w, const T* b, T* out,
                           hipStream_t stream) {
+    if (!shared_forward_chosen(s, sizeof(T))) return launch_direct<T>(s, in, off, mask, w, b, out, stream);
     SharedArgs<T> a{in, off, mask, w, b, out, s, (long)s.B * s.Ho * s.Wo, s.Cin / s.groups, s.Cout / s.groups,
                     s.Cin / s.og, 0, 0, 0, 0};
     const int ka = s.KH * s.KW;
-    // The shared kernel addresses each tensor with 32-bit byte offsets below 2^31 and its
-    // sampling positions with 32-bit integers; grid y is one workgroup column per group
-    // and channel tile.
-    const double limit = 2147483648.0;
-    const double in_bytes = (double)s.B * s.Cin * s.H * s.W * sizeof(T);
-    const double mask_bytes = (double)a.pixels * s.og * ka * sizeof(T);
-    const double weight_bytes = (double)s.Cout * a.cpg * ka * sizeof(T);
-    const double reach = std::max((double)s.Ho * s.sh + s.ph + (double)s.KH * s.dh,
-                                  (double)s.Wo * s.sw + s.pw + (double)s.KW * s.dw);
-    const bool fits = s.W >= 2 && in_bytes < limit && 2.0 * mask_bytes < limit && reach < 1e9 && s.ph > -1000000000 &&
-                      s.pw > -1000000000 && (double)s.groups * ((a.opg + 15) / 16) < 65536.0 &&
-                      weight_bytes < limit;
-    if (fits && (ka == 1 || ka == 2 || ka == 3 || ka == 4 || ka == 6 || ka == 9)) {
-        a.mask_bytes = (uint32_t)mask_bytes;
-        a.off_bytes = 2 * a.mask_bytes;
-        a.weight_bytes = (uint32_t)weight_bytes;
-        switch (ka) {
-            case 1: return launch_shared_ka<T, 1, 1>(a, stream);
-            case 2: return launch_shared_ka<T, 2, 1>(a, stream);
-            case 3: return launch_shared_ka<T, 3, 1>(a, stream);
-            case 4: return launch_shared_ka<T, 4, 1>(a, stream);
-            case 6: return launch_shared_ka<T, 6, 1>(a, stream);
-            default: break;
-        }
-        if (a.cpg % 8 == 0 && a.cpog % 8 == 0) return launch_shared_ka<T, 9, 8>(a, stream);
-        if (a.cpg % 4 == 0 && a.cpog % 4 == 0) return launch_shared_ka<T, 9, 4>(a, stream);
-        return launch_shared_ka<T, 9, 1>(a, stream);
+    a.mask_bytes = (uint32_t)((size_t)a.pixels * s.og * ka * sizeof(T));
+    a.off_bytes = 2 * a.mask_bytes;
+    a.weight_bytes = (uint32_t)((size_t)s.Cout * a.cpg * ka * sizeof(T));
+    switch (ka) {
+        case 1: return launch_shared_ka<T, 1, 1>(a, stream);
+        case 2: return launch_shared_ka<T, 2, 1>(a, stream);
+        case 3: return launch_shared_ka<T, 3, 1>(a, stream);
+        case 4: return launch_shared_ka<T, 4, 1>(a, stream);
+        case 6: return launch_shared_ka<T, 6, 1>(a, stream);
+        default: break;
     }
-    return launch_direct<T>(s, in, off, mask, w, b, out, stream);
+    switch (shared_item_channels(s)) {
+        case 8: return launch_shared_ka<T, 9, 8>(a, stream);
+        case 4: return launch_shared_ka<T, 9, 4>(a, stream);
+        default: return launch_shared_ka<T, 9, 1>(a, stream);
+    }
 }
 
 }  // namespace
+
+bool shared_forward_chosen(const KShape& s, size_t element) {
+    const int ka = s.KH * s.KW, opg = s.Cout / s.groups;
+    if (!(ka == 1 || ka == 2 || ka == 3 || ka == 4 || ka == 6 || ka == 9) || s.W < 2) return false;
+    // The kernel addresses each tensor with 32-bit byte offsets below 2^31 and its sampling
+    // positions with 32-bit integers; grid y is one workgroup column per group and channel
+    // tile, and a launch has fewer than 2^32 threads along x.
+    const double limit = 2147483648.0;
+    const double in_bytes = (double)s.B * s.Cin * s.H * s.W * element;
+    const double off_bytes = 2.0 * s.B * s.Ho * s.Wo * s.og * ka * element;
+    const double weight_bytes = (double)s.Cout * (s.Cin / s.groups) * ka * element;
+    const double reach = std::max((double)s.Ho * s.sh + s.ph + (double)s.KH * s.dh,
+                                  (double)s.Wo * s.sw + s.pw + (double)s.KW * s.dw);
+    if (in_bytes >= limit || off_bytes >= limit || weight_bytes >= limit || reach >= 1e9 || s.ph <= -1000000000 ||
+        s.pw <= -1000000000 || (double)s.groups * ((opg + 15) / 16) >= 65536.0)
+        return false;
+    const long tiles = shared_tiles(s);
+    const int waves = shared_split(tiles, opg).nw + shared_sampling_waves(ka, shared_item_channels(s));
+    return (double)(tiles / s.groups) * waves * 64 < 4294967296.0;
+}
 
 hipError_t launch_direct_f32(const KShape& s, const float* in, const float* off,
                              const float* mask, const float* w, const float* b, float* out,

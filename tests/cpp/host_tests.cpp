@@ -468,6 +468,22 @@ TEST(cpu, sharedKernelWeightLoadsStayInTheRun) {
         }
 }
 
+// A plain-weight layer [1][cin][h][w] -> cout of kernel x kernel taps, stride 1, same size.
+dcn::KShape plainLayer(int cin, int h, int w, int cout, int kernel, int groups = 1, int offsetGroups = 1) {
+    const int pad = kernel / 2;
+    return {1, cin, h, w, cout, h, w, kernel, kernel, pad, pad, 1, 1, 1, 1, groups, offsetGroups};
+}
+
+// A launch holds fewer than 2^32 threads along x. A 1x1 FP16 layer of three output channels
+// has 384 of them per 16 pixels on the shared-sample kernel: 178,956,970 pixels is the last
+// size that fits, and the tensors of the next ones are still within the library's limits.
+TEST(cpu, sharedKernelGridStaysBelowTheThreadLimit) {
+    EXPECT(dcn::shared_forward_chosen(plainLayer(8, 1000, 1000, 3, 1), 2));
+    EXPECT(dcn::shared_forward_chosen(plainLayer(2, 8192, 16384, 3, 1), 2));   // 134 M pixels
+    EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 8192, 21846, 3, 1), 2));  // 178,962,432
+    EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 15000, 16000, 1, 1), 2));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
