@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "dcn_device.hpp"
@@ -524,10 +525,13 @@ bool shared_forward_chosen(const KShape& s, size_t element) {
     const double in_bytes = (double)s.B * s.Cin * s.H * s.W * element;
     const double off_bytes = 2.0 * s.B * s.Ho * s.Wo * s.og * ka * element;
     const double weight_bytes = (double)s.Cout * (s.Cin / s.groups) * ka * element;
-    const double reach = std::max((double)s.Ho * s.sh + s.ph + (double)s.KH * s.dh,
-                                  (double)s.Wo * s.sw + s.pw + (double)s.KW * s.dw);
-    if (in_bytes >= limit || off_bytes >= limit || weight_bytes >= limit || reach >= 1e9 || s.ph <= -1000000000 ||
-        s.pw <= -1000000000 || (double)s.groups * ((opg + 15) / 16) >= 65536.0)
+    // Strides, dilations and pads may have either sign.
+    const auto reach = [](double out, double stride, double pad, double taps, double dilation) {
+        return out * std::fabs(stride) + std::fabs(pad) + taps * std::fabs(dilation);
+    };
+    if (in_bytes >= limit || off_bytes >= limit || weight_bytes >= limit ||
+        reach(s.Ho, s.sh, s.ph, s.KH, s.dh) >= 1e9 || reach(s.Wo, s.sw, s.pw, s.KW, s.dw) >= 1e9 ||
+        (double)s.groups * ((opg + 15) / 16) >= 65536.0)
         return false;
     const long tiles = shared_tiles(s);
     const int waves = shared_split(tiles, opg).nw + shared_sampling_waves(ka, shared_item_channels(s));

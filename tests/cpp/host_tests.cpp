@@ -484,6 +484,25 @@ TEST(cpu, sharedKernelGridStaysBelowTheThreadLimit) {
     EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 15000, 16000, 1, 1), 2));
 }
 
+// The shared-sample kernel's sampling positions are 32-bit integers, the other kernel's 64-bit:
+// strides and dilations of either sign that could leave 32 bits take the other one.
+TEST(cpu, sharedKernelPositionsStayInRange) {
+    for (const int sign : {1, -1}) {
+        dcn::KShape s = plainLayer(64, 32, 32, 64, 3);
+        s.sh = s.sw = sign * 2;
+        s.dh = s.dw = sign * 3;
+        EXPECT(dcn::shared_forward_chosen(s, 2));
+        s.sh = sign * 100000000;
+        EXPECT(!dcn::shared_forward_chosen(s, 2));
+        s.sh = 1;
+        s.dw = sign * 1000000000;
+        EXPECT(!dcn::shared_forward_chosen(s, 4));
+        s.dw = 1;
+        s.ph = sign * 1000000000;
+        EXPECT(!dcn::shared_forward_chosen(s, 4));
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
