@@ -534,8 +534,26 @@ bool shared_forward_chosen(const KShape& s, size_t element) {
         (double)s.groups * ((opg + 15) / 16) >= 65536.0)
         return false;
     const long tiles = shared_tiles(s);
-    const int waves = shared_split(tiles, opg).nw + shared_sampling_waves(ka, shared_item_channels(s));
-    return (double)(tiles / s.groups) * waves * 64 < 4294967296.0;
+    const SharedSplit split = shared_split(tiles, opg);
+    const int items = shared_item_channels(s);
+    if ((double)(tiles / s.groups) * (split.nw + shared_sampling_waves(ka, items)) * 64 >= 4294967296.0) return false;
+    // Groups of few channels: a workgroup samples 16 input channels and sums 16 output channels
+    // or more however few the group has, so depthwise layers and their like run one thread per
+    // output, where there are enough of them. Fitted to both kernels' times over 946 layers
+    // (FP32 and FP16; 1, 4, 9 taps; 256 to 262,144 pixels; 1 to 128 channels a group): the
+    // shared-sample kernel 1.3 ns per workgroup, stage and tap (0.6 with items of eight
+    // channels), the other 5 ps per sample and output (FP16 4.5) or, with few outputs, 0.6 us
+    // per sample of one. us per call, shared / one thread per output, FP16: 64 groups of 1 -> 1
+    // on 64x64 221 / 12.6 and on 180x320 3182 / 207, 3 groups of 2 -> 2 there 158 / 44, 16
+    // of 4 -> 4 on 64x64 47.7 / 41.6, 3 -> 3 on 64x64 5.9 / 20.9, 8 groups of 4 -> 8 there
+    // 25.7 / 40.6. From two whole stages on the samples' sharing wins in nearly all.
+    const int cpg = s.Cin / s.groups, oc = 4 * split.nw * split.ocl;
+    if (cpg >= 2 * kSharedCh) return true;
+    const double samples = (double)s.B * s.Ho * s.Wo * s.Cout * cpg * ka;
+    const double direct_us = std::max(0.6 * cpg * ka, samples * (element == 2 ? 4.5e-6 : 5e-6));
+    const double shared_us = (double)tiles * ((opg + oc - 1) / oc) * ((cpg + kSharedCh - 1) / kSharedCh) * ka *
+                             (items == 8 ? 0.6e-3 : 1.3e-3);
+    return shared_us <= direct_us;
 }
 
 hipError_t launch_direct_f32(const KShape& s, const float* in, const float* off,

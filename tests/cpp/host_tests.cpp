@@ -478,8 +478,7 @@ dcn::KShape plainLayer(int cin, int h, int w, int cout, int kernel, int groups =
 // has 384 of them per 16 pixels on the shared-sample kernel: 178,956,970 pixels is the last
 // size that fits, and the tensors of the next ones are still within the library's limits.
 TEST(cpu, sharedKernelGridStaysBelowTheThreadLimit) {
-    EXPECT(dcn::shared_forward_chosen(plainLayer(8, 1000, 1000, 3, 1), 2));
-    EXPECT(dcn::shared_forward_chosen(plainLayer(2, 8192, 16384, 3, 1), 2));   // 134 M pixels
+    EXPECT(dcn::shared_forward_chosen(plainLayer(32, 1000, 1000, 3, 1), 2));
     EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 8192, 21846, 3, 1), 2));  // 178,962,432
     EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 15000, 16000, 1, 1), 2));
 }
@@ -500,6 +499,22 @@ TEST(cpu, sharedKernelPositionsStayInRange) {
         s.dw = 1;
         s.ph = sign * 1000000000;
         EXPECT(!dcn::shared_forward_chosen(s, 4));
+    }
+}
+
+// Layers whose groups are much smaller than the shared-sample kernel's 16 x 16 channels run one
+// thread per output, unless that leaves too few threads.
+TEST(cpu, sharedKernelOnlyWhereGroupsFillIt) {
+    for (const size_t element : {2, 4}) {
+        EXPECT(!dcn::shared_forward_chosen(plainLayer(64, 64, 64, 64, 3, 64), element));       // depthwise
+        EXPECT(!dcn::shared_forward_chosen(plainLayer(64, 180, 320, 64, 3, 64, 64), element));
+        EXPECT(!dcn::shared_forward_chosen(plainLayer(6, 180, 320, 6, 3, 3), element));        // 2 -> 2
+        EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 512, 512, 3, 1), element));
+        EXPECT(dcn::shared_forward_chosen(plainLayer(3, 64, 64, 3, 3), element));              // few outputs
+        EXPECT(dcn::shared_forward_chosen(plainLayer(32, 64, 64, 64, 3, 8), element));         // 4 -> 8
+        EXPECT(dcn::shared_forward_chosen(plainLayer(128, 64, 64, 128, 3, 16, 16), element));  // 8 -> 8
+        EXPECT(dcn::shared_forward_chosen(plainLayer(128, 64, 64, 64, 3, 1, 16), element));
+        EXPECT(dcn::shared_forward_chosen(plainLayer(128, 512, 512, 1, 3, 1, 16), element));
     }
 }
 

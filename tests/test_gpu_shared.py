@@ -25,6 +25,7 @@ SHAPES = [
     ((1, 4, 9, 10, 1, 9, 10, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1), 3.0),       # 36 weights in all: less than a stage
     ((1, 16, 9, 10, 1, 9, 10, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1), 3.0),      # one output channel, one whole stage
     ((1, 33, 9, 10, 2, 9, 10, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1), 3.0),      # two whole stages and one channel
+    ((2, 24, 33, 40, 24, 33, 40, 3, 3, 1, 1, 1, 1, 1, 1, 24, 24), 3.0),  # depthwise: the one-thread kernel
 ]
 
 
