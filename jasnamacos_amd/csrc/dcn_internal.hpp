@@ -257,15 +257,15 @@ struct ConvEnds {
     const void *res1, *res2, *out, *out2;  // null: absent
     int res1_layout, res2_layout, out_layout;
 };
-bool conv_wide_chosen(int height, int width, int images, const ConvEnds& ends, int chunks = 1);
+bool conv_wide_chosen(int height, int width, int images, const ConvEnds& ends);
 hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk1, const float* bias1,
                                     int act1, const void* wpk2, const float* bias2, int act2, float slope,
                                     const uint16_t* res1, int res1_layout, const uint16_t* res2, int res2_layout,
                                     uint16_t* out, int out_layout, hipStream_t stream, int res2_coff,
                                     const ConvBatch& batch, uint16_t* out2_cb8);
 // One conv on larger tiles (dcn_kernels_conv_wide.hip), for the body's input channel counts
-// and output channels in multiples of four; launch_conv3x3 runs it where conv_wide_chosen.
-bool conv_wide_supported(const ConvGeometry& g);
+// and output channels in multiples of four; launch_conv3x3 runs it where conv3x3_wide_chosen.
+bool conv3x3_wide_chosen(const ConvGeometry& g, const void* x_cb8, int images, const ConvEnds& ends);
 hipError_t launch_conv3x3_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk, const float* bias, int act,
                                float slope, const uint16_t* res1, int res1_layout, const uint16_t* res2,
                                int res2_layout, uint16_t* out, int out_layout, hipStream_t stream, int res2_coff,

@@ -1366,9 +1366,7 @@ hipError_t launch_conv3x3(const ConvGeometry& g, const void* x_cb8, const void* 
                           const float* bias, int act, float slope, const uint16_t* res1,
                           int res1_layout, const uint16_t* res2, int res2_layout, uint16_t* out,
                           int out_layout, hipStream_t stream, int res2_coff, const ConvBatch& batch) {
-    if (conv_wide_supported(g) && batch.images >= 1 &&
-        conv_wide_chosen(g.h, g.w, batch.images, {res1, res2, out, nullptr, res1_layout, res2_layout, out_layout},
-                         g.chunks))
+    if (conv3x3_wide_chosen(g, x_cb8, batch.images, {res1, res2, out, nullptr, res1_layout, res2_layout, out_layout}))
         return launch_conv3x3_wide(g, x_cb8, wpk, bias, act, slope, res1, res1_layout, res2, res2_layout, out,
                                    out_layout, stream, res2_coff, batch);
     ConvArgs a{};

@@ -531,19 +531,28 @@ static long wide_tiles(int height, int width, int images, int th) {
     return (long)images * ((height + th - 1) / th) * ((width + kWideTW - 1) / kWideTW);
 }
 
+// The wide kernels read and write four channels of a CB8 unit at once: those tensors must be
+// 8-byte aligned.
+static bool ends_aligned(const ConvEnds& t) {
+    const auto ok = [](const void* p, int layout) { return layout != kLayoutCB8 || (uintptr_t)p % 8 == 0; };
+    return ok(t.res1, t.res1_layout) && ok(t.res2, t.res2_layout) && ok(t.out, t.out_layout) && ok(t.out2, kLayoutCB8);
+}
+static long tiles_2x8(int height, int width, int images) { return (long)images * ((height + 1) / 2) * ((width + 7) / 8); }
+
 // Up to 256 tiles of 2 x 8 pixels the 16-pixel kernels of dcn_kernels_conv.hip run as one
 // workgroup per CU and are faster (a pair at 64x64, 256 of them: 6.7 against 7.1 us; at
-// 64x72, 288: 11.5 against 7.5; 320 -> 64 there 10.7 against 10.0). The wide kernels read and write four channels of a CB8 unit
-// at once: those tensors must be 8-byte aligned.
-bool conv_wide_chosen(int height, int width, int images, const ConvEnds& t, int chunks) {
-    const auto ok = [](const void* p, int layout) { return layout != kLayoutCB8 || (uintptr_t)p % 8 == 0; };
-    return (long)images * ((height + 1) / 2) * ((width + 7) / 8) * chunks > 256 && ok(t.res1, t.res1_layout) &&
-           ok(t.res2, t.res2_layout) && ok(t.out, t.out_layout) && ok(t.out2, kLayoutCB8);
+// 64x72, 288: 11.5 against 7.5).
+bool conv_wide_chosen(int height, int width, int images, const ConvEnds& t) {
+    return tiles_2x8(height, width, images) > 256 && ends_aligned(t);
 }
 
-bool conv_wide_supported(const ConvGeometry& g) {
+// The same for one conv (320 -> 64 at 64x72 10.7 against 10.0 us). Its input comes by 16-byte
+// LDS DMA and must be 16-byte aligned.
+bool conv3x3_wide_chosen(const ConvGeometry& g, const void* x_cb8, int images, const ConvEnds& t) {
     const int cb = g.cb;
-    return (cb == 8 || cb == 16 || cb == 24 || cb == 25 || cb == 32 || cb == 40) && g.cout % 4 == 0;
+    const bool supported = (cb == 8 || cb == 16 || cb == 24 || cb == 25 || cb == 32 || cb == 40) && g.cout % 4 == 0;
+    return supported && images >= 1 && tiles_2x8(g.h, g.w, images) * g.chunks > 256 && (uintptr_t)x_cb8 % 16 == 0 &&
+           ends_aligned(t);
 }
 
 hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk1, const float* bias1,

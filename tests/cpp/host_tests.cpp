@@ -518,6 +518,21 @@ TEST(cpu, sharedKernelOnlyWhereGroupsFillIt) {
     }
 }
 
+// Whether one conv cin -> cout on h x w runs the large-tile kernel, its CB8 input `shift` bytes
+// past an aligned address.
+bool convWide(int cin, int cout, int h, int w, size_t shift = 0, int images = 1) {
+    const auto at = [](size_t address) { return reinterpret_cast<const void*>(address); };
+    const dcn::ConvEnds ends{nullptr, nullptr, at(4096), nullptr, 0, 0, DCN_TENSOR_CB8};
+    return dcn::conv3x3_wide_chosen(dcn::conv_geometry(cin, cout, h, w), at(8192 + shift), images, ends);
+}
+
+// The large-tile conv copies 16-byte units of its input by DMA: other alignments take the
+// 16-pixel kernel.
+TEST(cpu, largeTileConvNeedsAlignedInput) {
+    EXPECT(convWide(128, 64, 180, 320));
+    for (const size_t shift : {2, 4, 8}) EXPECT(!convWide(128, 64, 180, 320, shift));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {

@@ -118,3 +118,23 @@ def test_wide_conv_same_bits(gpu_ctx, torch, cin, cout, h, w, act, residuals, la
     assert np.array_equal(np.isnan(a), np.isnan(b))
     assert np.array_equal(got[~np.isnan(b)], want[~np.isnan(b)])
     assert np.isfinite(a).mean() > 0.9
+
+
+@pytest.mark.parametrize("cin", [64, 196])
+def test_wide_conv_input_alignment(gpu_ctx, torch, cin):
+    """An input 8 bytes past a 16-byte boundary (the 16-pixel kernel): the same bits."""
+    h, w = 67, 131
+    rng = np.random.default_rng(cin)
+    print("case: conv input alignment", cin, flush=True)
+    f16 = lambda *s, std=1.0: br.f16(rng.normal(0, std, s))  # noqa: E731
+    x = br.to_cb8(f16(cin, h, w), cin, h, w)
+    conv = gpu_ctx.conv3x3(cin, 64, h, w, _dev(torch, f16(64, cin, 3, 3, std=0.04)), _dev(torch, f16(64, std=0.1)))
+    outs = []
+    for shift in (0, 4):
+        xd = _operand(torch, x, shift)
+        out = _placed(torch, 8 * (h + 4) * (w + 4) * 8, 0)
+        conv.run_dev(xd, out, CB8, activation=1)
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    conv.free()
+    assert np.array_equal(outs[0], outs[1]) and outs[0].any()
