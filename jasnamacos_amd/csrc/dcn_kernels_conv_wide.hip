@@ -546,13 +546,22 @@ bool conv_wide_chosen(int height, int width, int images, const ConvEnds& t) {
     return tiles_2x8(height, width, images) > 256 && ends_aligned(t);
 }
 
-// The same for one conv (320 -> 64 at 64x72 10.7 against 10.0 us). Its input comes by 16-byte
-// LDS DMA and must be 16-byte aligned.
+// One conv over one image: both kernels' times by their workgroups, `flat` of 16 pixels and `wide` of
+// 4 x 16, timed for 11 channel counts at 294 sizes. Up to 512 flat ones (two per CU) stay one round;
+// the wide kernel beats that only with more than 64 channels to read, and one workgroup per CU
+// itself (us flat / wide: 64x72 320 -> 64 10.1 / 9.9, 128 -> 64 7.4 / 6.1, 64 -> 64 4.6 / 5.0). Beyond,
+// by the time of a workgroup of each: a map narrower than 4 to 8 columns leaves most of a
+// 16-wide tile empty (1030x3 320 -> 64 7.1 / 15.0; 2600x4 64 -> 64 6.6 / 8.6; 1696x5 256 -> 64
+// 12.1 / 12.6, 128 -> 64 10.6 / 8.2). Over several images: as the pair, whose workgroups it shares.
+// The input comes by 16-byte LDS DMA and must be 16-byte aligned.
 bool conv3x3_wide_chosen(const ConvGeometry& g, const void* x_cb8, int images, const ConvEnds& t) {
     const int cb = g.cb;
     const bool supported = (cb == 8 || cb == 16 || cb == 24 || cb == 25 || cb == 32 || cb == 40) && g.cout % 4 == 0;
-    return supported && images >= 1 && tiles_2x8(g.h, g.w, images) * g.chunks > 256 && (uintptr_t)x_cb8 % 16 == 0 &&
-           ends_aligned(t);
+    if (!supported || images < 1 || (uintptr_t)x_cb8 % 16 != 0 || !ends_aligned(t)) return false;
+    if (images > 1) return tiles_2x8(g.h, g.w, images) * g.chunks > 256;
+    const long flat = ((long)g.h * g.w + 15) / 16 * g.chunks, wide = wide_tiles(g.h, g.w, 1, 4) * g.chunks;
+    if (flat <= 512) return flat > 256 && cb > 8 && wide <= 256;
+    return wide * (cb == 8 ? 1.4 : cb <= 25 ? 1.0 : 1.8) <= (double)flat;
 }
 
 hipError_t launch_conv3x3_pair_wide(const ConvGeometry& g, const void* x_cb8, const void* wpk1, const float* bias1,

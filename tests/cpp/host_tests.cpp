@@ -533,6 +533,21 @@ TEST(cpu, largeTileConvNeedsAlignedInput) {
     for (const size_t shift : {2, 4, 8}) EXPECT(!convWide(128, 64, 180, 320, shift));
 }
 
+// Maps much narrower than a 16-pixel-wide tile, and small maps of 64 channels, are faster on the
+// 16-pixel kernel; batches go by their tiles.
+TEST(cpu, largeTileConvByWorkgroups) {
+    for (const int cin : {64, 128, 196, 320}) {
+        EXPECT(!convWide(cin, 64, 64, 64));
+        EXPECT(convWide(cin, 64, 64, 72) == (cin > 64));
+        EXPECT(convWide(cin, 64, 180, 320));
+        EXPECT(!convWide(cin, 64, 1030, 3));
+        EXPECT(!convWide(cin, 64, 20000, 2));
+        EXPECT(convWide(cin, 64, 2600, 8));
+        EXPECT(convWide(cin, 64, 64, 4, 0, 64));
+    }
+    EXPECT(!convWide(64, 64, 2600, 4) && !convWide(64, 432, 32, 32) && convWide(64, 432, 64, 64));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {

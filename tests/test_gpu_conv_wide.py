@@ -90,7 +90,8 @@ CHANNELS = [(64, 64), (128, 64), (192, 20), (196, 64), (256, 64), (320, 64), (61
 
 
 @pytest.mark.parametrize("cin,cout", CHANNELS, ids=lambda v: str(v))
-@pytest.mark.parametrize("h,w,act,residuals,layout", [(67, 131, 1, 0, CB8), (90, 401, 2, 2, CB8), (5, 1500, 0, 1, NCHW)])
+@pytest.mark.parametrize("h,w,act,residuals,layout", [(67, 131, 1, 0, CB8), (90, 401, 2, 2, CB8), (5, 1500, 0, 1, NCHW),
+                                                      (1100, 8, 1, 2, CB8)])
 def test_wide_conv_same_bits(gpu_ctx, torch, cin, cout, h, w, act, residuals, layout):
     """One conv on tiles of 4 and 8 rows against the 16-pixel-tile kernel."""
     rng = np.random.default_rng(cin * 7 + cout + h)
