@@ -47,7 +47,12 @@ dcn::FusedConfig choose_config(dcn::FusedConfig o, const dcn::FusedGeometry& g, 
     // one pass per window).
     // The same holds for the exact sampler (the reference's FP32 blend, about 104 VALU per
     // sample): C3 67.4 against 67.6 us for the window kernel, C5 71.9 against 73.2.
-    if (o.variant == 0 && tile_ok && (g.m + 31) / 32 > 1024) o.variant = dcn::kVariantTile;
+    // Below, the tile kernel still takes the time of its one round of workgroups, the narrow
+    // kernel one by the pixel. Fast sampler, us narrow / tile: 768 tiles of 32 pixels (128x192)
+    // 46.6 / 52.1, 896 (7 x 64x64) 51.5 / 51.5 and with 32 px flows 55.8 / 60.4, 951 (181x168)
+    // 63.5 / 55.6, 1024 (8 x 64x64) 58.1 / 50.6. Exact sampler at 1024: 60.7 / 69.8.
+    const long long tile_above = o.sampler == dcn::kSamplerExact ? 1024 : 928;
+    if (o.variant == 0 && tile_ok && (g.m + 31) / 32 > tile_above) o.variant = dcn::kVariantTile;
     // A shape the tile variant does not cover gets the automatic choice below, with only
     // the sampler pinned.
     if (o.variant == dcn::kVariantTile) {
@@ -161,13 +166,18 @@ dcn_status fused_prepacked_dev(dcn_context* ctx, const dcn_shape* shape, const v
     // as FP16 does; above, LDS windows over 4 x 32 tiles where the shape allows them, else
     // the register variant with 64-pixel tiles over 4 K-waves.
     const long long tiles32 = (g.m + 31) / 32;
+    // Up to 1024 tiles the automatic choice of the tile kernel, which copies offsets and masks in
+    // 16-byte pieces, needs them 16-byte aligned, and no clock buffer set (it would have
+    // to hold this launch's stamps); the narrow kernel it stands in for needs neither.
+    const bool tile_pinned = ctx->fused_override.variant == dcn::kVariantTile || tiles32 > 1024;
+    const bool tile_ready = tile_pinned || (((uintptr_t)d_offset | (uintptr_t)d_mask) % 16 == 0 && !ctx->tile_clock);
     const bool bf16_window = packed->weights_group != nullptr && dcn::window_supported(*shape);
     const dcn::FusedConfig cfg =
         bf16 ? (tiles32 <= 1024 ? dcn::FusedConfig{dcn::kVariantNarrow, 1, 12, dcn::kSamplerBf16}
                 : bf16_window   ? dcn::FusedConfig{dcn::kVariantWindow, 4, 4, dcn::kSamplerBf16}
                                 : dcn::FusedConfig{dcn::kVariantRegister, 2, 4, dcn::kSamplerBf16})
              : choose_config(ctx->fused_override, g, *shape, packed->weights_group != nullptr && dcn::window_supported(*shape),
-                             packed->weights_tile != nullptr && dcn::tile_supported(*shape));
+                             tile_ready && packed->weights_tile != nullptr && dcn::tile_supported(*shape));
     if (!config_supported(cfg, g))
         return fail(ctx, DCN_INVALID_ARGUMENT,
                     "unsupported fused config (variant " + std::to_string(cfg.variant) + ", mt " +
