@@ -166,11 +166,10 @@ dcn_status fused_prepacked_dev(dcn_context* ctx, const dcn_shape* shape, const v
     // as FP16 does; above, LDS windows over 4 x 32 tiles where the shape allows them, else
     // the register variant with 64-pixel tiles over 4 K-waves.
     const long long tiles32 = (g.m + 31) / 32;
-    // Up to 1024 tiles the automatic choice of the tile kernel, which copies offsets and masks in
-    // 16-byte pieces, needs them 16-byte aligned, and no clock buffer set (it would have
-    // to hold this launch's stamps); the narrow kernel it stands in for needs neither.
+    // Up to 1024 tiles the automatic choice of the tile kernel needs no clock buffer set (it
+    // would have to hold this launch's stamps); the narrow kernel it stands in for does not.
     const bool tile_pinned = ctx->fused_override.variant == dcn::kVariantTile || tiles32 > 1024;
-    const bool tile_ready = tile_pinned || (((uintptr_t)d_offset | (uintptr_t)d_mask) % 16 == 0 && !ctx->tile_clock);
+    const bool tile_ready = tile_pinned || !ctx->tile_clock;
     const bool bf16_window = packed->weights_group != nullptr && dcn::window_supported(*shape);
     const dcn::FusedConfig cfg =
         bf16 ? (tiles32 <= 1024 ? dcn::FusedConfig{dcn::kVariantNarrow, 1, 12, dcn::kSamplerBf16}

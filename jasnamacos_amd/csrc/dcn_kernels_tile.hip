@@ -297,6 +297,42 @@ __device__ __forceinline__ void tile_copy_offsets(const TileArgs& a, __amdgpu_bu
     }
 }
 
+// The same for offsets or masks off 16-byte alignment, which the DMA's 16-byte pieces need:
+// through registers, by loads of any alignment (chunks past a tensor's end are zero, as
+// the DMA's range check leaves them). Each stage waits for the loads before their LDS writes.
+// us aligned / not, narrow kernel in brackets: 8 x 64x64 42.5 / 51.8 (56.7 / 58.3), with 32 px
+// flows 59.9 / 67.0 (62.3 / 62.7), 16 x 64x64 57.6 / 66.8.
+template <int TW>
+__device__ __forceinline__ void tile_load_offsets(const TileArgs& a, int b, int ty, int tx, int st, uint8_t* dst,
+                                                  int wave, int lane) {
+    constexpr int NW = kTileWaves;
+    constexpr int TH = kTilePix / TW;
+    constexpr int kRowChunks = TW / 8;
+    constexpr int kChunks = kTileOffCh * (kTilePix / 8);
+    constexpr int kOffChunks = 36 * (kTilePix / 8);
+    constexpr int kIter = (kChunks + 64 * NW - 1) / (64 * NW);
+    const int rem = lane % 16;
+    const int y = min(ty * TH + rem / kRowChunks, a.Ho - 1);
+    const int x = tx * TW + (rem % kRowChunks) * 8;
+    u32x4 q[kIter];
+#pragma unroll
+    for (int k = 0; k < kIter; ++k) {
+        const int c = (wave + k * NW) * 64 + lane;  // chunk: channel c / 16
+        const bool is_off = c < kOffChunks;
+        const uint32_t ch = is_off ? (uint32_t)(b * 2 * a.G * 9 + 36 * st) + c / 16
+                                   : (uint32_t)(b * a.G * 9 + 18 * st) + c / 16 - 36;
+        const uint32_t at = (ch * (uint32_t)a.HWo + (uint32_t)(y * a.Wo + x)) * 2u;  // bytes
+        q[k] = u32x4{0u, 0u, 0u, 0u};
+        if (c < kChunks && at + 16u <= (is_off ? a.off_bytes : a.msk_bytes))
+            __builtin_memcpy(&q[k], reinterpret_cast<const uint8_t*>(is_off ? a.off : a.msk) + at, 16);
+    }
+#pragma unroll
+    for (int k = 0; k < kIter; ++k) {
+        const int c = (wave + k * NW) * 64 + lane;
+        if (c < kChunks) *reinterpret_cast<u32x4*>(dst + c * 16) = q[k];
+    }
+}
+
 // A tile's estimate for the pair placement: the extent of its clamped corner positions
 // (floor of the sample position, clamped like the stage loop's corners) for group 0's
 // centre tap over every pixel, (rows + 3) x (columns + 3). It is the window box of one
@@ -417,7 +453,9 @@ __device__ __forceinline__ int tile_pair_slot(const TileArgs& a, __amdgpu_buffer
     return band0 + (loc ^ 32);
 }
 
-template <int NB, int TW, bool EXACT, bool PAIR>
+// DMA: offsets and masks 16-byte aligned, copied by LDS DMA (else through registers, with the
+// fixed placement).
+template <int NB, int TW, bool EXACT, bool PAIR, bool DMA = true>
 __global__ __launch_bounds__(64 * kTileWaves, 2) void tile_kernel(TileArgs a) {
     constexpr int NW = kTileWaves;
     constexpr int RPW = 32 / TW;  // tile rows per 32-pixel segment
@@ -452,7 +490,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void tile_kernel(TileArgs a) {
     // in the window buffer.
     const bool pair_plan = PAIR && a.plan && band_n == 64;
     const int tile = pair_plan ? tile_pair_slot<NB, TW>(a, orr, mr, wr, band0, loc, offs, lds)
-                               : band0 + (a.plan && band_n > 32 && band_n < 64
+                               : band0 + (DMA && a.plan && band_n > 32 && band_n < 64
                                               ? tile_band_slot<TW>(a, orr, band0, band_n, loc,
                                                                    reinterpret_cast<float*>(lds))
                                               : loc);
@@ -497,7 +535,10 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void tile_kernel(TileArgs a) {
             ybf[s][t] = (float)(ybi[s] + t * a.dh);
             xbf[s][t] = (float)(xbi[s] + t * a.dw);
         }
-    auto copy_offsets = [&](int st) { tile_copy_offsets<TW>(a, orr, mr, b, ty, tx, st, offs, wave, lane); };
+    auto copy_offsets = [&](int st) {
+        if constexpr (DMA) tile_copy_offsets<TW>(a, orr, mr, b, ty, tx, st, offs, wave, lane);
+        else tile_load_offsets<TW>(a, b, ty, tx, st, offs, wave, lane);
+    };
 
     // Window geometry of a stage (wave-uniform): origin, size in units, LDS placement.
     struct Win {
@@ -934,9 +975,9 @@ __global__ __launch_bounds__(256) void tile_prepack_kernel(const uint16_t* __res
     wpk[gid] = v;
 }
 
-template <int NB, int TW, bool EXACT, bool PAIR>
+template <int NB, int TW, bool EXACT, bool PAIR, bool DMA = true>
 hipError_t launch_tile_p(const TileArgs& a, hipStream_t stream) {
-    auto kernel = &tile_kernel<NB, TW, EXACT, PAIR>;
+    auto kernel = &tile_kernel<NB, TW, EXACT, PAIR, DMA>;
     const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kTileLds);
     if (attr != hipSuccess) return attr;
     const unsigned grid = (unsigned)(((a.tiles + 7) / 8) * 8);
@@ -948,6 +989,7 @@ hipError_t launch_tile_p(const TileArgs& a, hipStream_t stream) {
 // tiles (every CU of an XCD runs two); every other shape runs the kernel without it.
 template <int NB, int TW, bool EXACT>
 hipError_t launch_tile_t(const TileArgs& a, hipStream_t stream) {
+    if (((uintptr_t)a.off | (uintptr_t)a.msk) % 16 != 0) return launch_tile_p<NB, TW, EXACT, false, false>(a, stream);
     return a.plan && (a.tiles + 7) / 8 == 64 ? launch_tile_p<NB, TW, EXACT, true>(a, stream)
                                              : launch_tile_p<NB, TW, EXACT, false>(a, stream);
 }
