@@ -286,7 +286,8 @@ dcn_status dcn_forward_f16_prepacked_noalloc_dev(dcn_context* ctx, const dcn_sha
  * others two (33-63 tiles per band), and where every CU runs two (64 tiles per band) a
  * heavy tile goes to the slot dispatched first; ks = 1: fixed placement; the outputs are
  * the same bits either way; the automatic choice for problems of more than 1024 tiles of 32
- * pixels, and with the fast sampler of more than 928 where no clock buffer is set; offsets
+ * pixels, and with the fast sampler of more than 928 where neither mt nor ks is
+ * pinned and no clock buffer is set; offsets
  * and masks off 16-byte alignment are copied through registers: the same bits). sampler: 0 = reference arithmetic
  * (FP32 bilinear in the reference's association, half(sampled*mask): the im2col
  * values of deform_conv2d_fp16_jasna_gather bit for bit), 1 = fast (mask folded into

@@ -50,8 +50,10 @@ dcn::FusedConfig choose_config(dcn::FusedConfig o, const dcn::FusedGeometry& g, 
     // Below, the tile kernel still takes the time of its one round of workgroups, the narrow
     // kernel one by the pixel. Fast sampler, us narrow / tile: 768 tiles of 32 pixels (128x192)
     // 46.6 / 52.1, 896 (7 x 64x64) 51.5 / 51.5 and with 32 px flows 55.8 / 60.4, 951 (181x168)
-    // 63.5 / 55.6, 1024 (8 x 64x64) 58.1 / 50.6. Exact sampler at 1024: 60.7 / 69.8.
-    const long long tile_above = o.sampler == dcn::kSamplerExact ? 1024 : 928;
+    // 63.5 / 55.6, 1024 (8 x 64x64) 58.1 / 50.6. Exact sampler at 1024: 60.7 / 69.8. A pinned
+    // mt or ks is one of the narrow kernel's up to 1024 tiles.
+    const bool pinned = o.mt > 0 || o.ks > 0;
+    const long long tile_above = o.sampler == dcn::kSamplerExact || pinned ? 1024 : 928;
     if (o.variant == 0 && tile_ok && (g.m + 31) / 32 > tile_above) o.variant = dcn::kVariantTile;
     // A shape the tile variant does not cover gets the automatic choice below, with only
     // the sampler pinned.

@@ -79,3 +79,21 @@ def test_pinned_tile_widths_take_any_alignment(gpu_ctx, dcn, torch, mt):
             assert np.array_equal(call.run(off, msk), want), (off, msk)
     finally:
         gpu_ctx.set_fused_config(0, 0, -1, 0)
+
+
+@pytest.mark.parametrize("mt,ks", [(1, 0), (0, 12), (1, 12), (0, 8)])
+def test_pinned_narrow_settings_keep_the_narrow_kernel(gpu_ctx, dcn, torch, mt, ks):
+    """The automatic variant with the narrow kernel's mt or ks pinned, at 929 to 1024 tiles: the
+    narrow kernel with those settings, as at every smaller size."""
+    print("case: pinned narrow settings", mt, ks, flush=True)
+    call = Call(torch, gpu_ctx, dcn, 8, 64, 64)
+    outs = []
+    try:
+        for variant in (0, dcn.VARIANT_NARROW):
+            gpu_ctx.set_fused_config(mt, ks, -1, variant)
+            cfg = gpu_ctx.get_fused_config(call.shape)
+            assert (cfg["variant"], cfg["mt"], cfg["ks"]) == (dcn.VARIANT_NARROW, 1, ks or 12)
+            outs.append(call.run())
+        assert np.array_equal(outs[0], outs[1])
+    finally:
+        gpu_ctx.set_fused_config(0, 0, -1, 0)
