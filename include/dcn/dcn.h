@@ -286,11 +286,10 @@ dcn_status dcn_forward_f16_prepacked_noalloc_dev(dcn_context* ctx, const dcn_sha
  * others two (33-63 tiles per band), and where every CU runs two (64 tiles per band) a
  * heavy tile goes to the slot dispatched first; ks = 1: fixed placement; the outputs are
  * the same bits either way; the automatic choice for problems of more than 1024 tiles of 32
- * pixels, and with the fast sampler of more than 928 where neither mt nor ks is
- * pinned and no clock buffer is set; offsets
- * and masks off 16-byte alignment are copied through registers: the same bits). sampler: 0 = reference arithmetic
- * (FP32 bilinear in the reference's association, half(sampled*mask): the im2col
- * values of deform_conv2d_fp16_jasna_gather bit for bit), 1 = fast (mask folded into
+ * pixels, and with the fast sampler of more than 928 where neither mt nor ks is pinned;
+ * offsets and masks off 16-byte alignment are copied through registers: the same bits).
+ * sampler: 0 = reference arithmetic (FP32 bilinear in the reference's association,
+ * half(sampled*mask): the im2col values of deform_conv2d_fp16_jasna_gather bit for bit), 1 = fast (mask folded into
  * the bilinear weights, packed-FP16 blend). mt = 32-pixel row blocks per tile (1, 2),
  * ks = waves per workgroup (register: 2, 4, 8; staged: 8, 16). 0 / -1 = automatic.
  * The setting applies to the FP16 prepacked forwards; the BF16 forwards choose their
@@ -299,8 +298,9 @@ dcn_status dcn_forward_f16_prepacked_noalloc_dev(dcn_context* ctx, const dcn_sha
  * No counterpart in the reference (its tile size is the compile-time
  * fusedGEMMRowsPerTile, MetalShader.swift:2). */
 dcn_status dcn_set_fused_config(dcn_context* ctx, int variant, int mt, int ks, int sampler);
-/* The configuration the next FP16 fused call on `shape` would use. ctx may be null: the
- * automatic choice without an override (no device is touched). */
+/* The configuration the next FP16 fused call on `shape` would use, with weights prepacked
+ * for it, whatever the pointers' alignment. ctx may be null: the automatic choice without an
+ * override (no device is touched). */
 dcn_status dcn_get_fused_config(dcn_context* ctx, const dcn_shape* shape, int* variant, int* mt,
                                 int* ks, int* sampler);
 
@@ -317,7 +317,8 @@ dcn_status dcn_launch_floor_dev(dcn_context* ctx, int workgroups, int threads, i
  * issued its output stores; HW_ID and XCC_ID are the hardware registers of that name
  * (bits 15:8 of HW_ID and XCC_ID together name the CU). Workgroups without a tile write nothing, so the caller clears the buffer.
  * `count` is in uint64 elements; a tile launch needs 4 x its workgroup count
- * (8 x ceil(tiles / 8)) and fails with DCN_INVALID_ARGUMENT when the buffer is smaller.
+ * (8 x ceil(tiles / 8)) and fails with DCN_INVALID_ARGUMENT when the buffer is smaller
+ * (up to 1024 tiles of 32 pixels without the variant pinned: goes on without stamps).
  * A null d_clock turns the stamps off. No counterpart in the reference. */
 dcn_status dcn_set_tile_clock_dev(dcn_context* ctx, void* d_clock, size_t count);
 

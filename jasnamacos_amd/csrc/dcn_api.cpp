@@ -168,25 +168,25 @@ dcn_status fused_prepacked_dev(dcn_context* ctx, const dcn_shape* shape, const v
     // as FP16 does; above, LDS windows over 4 x 32 tiles where the shape allows them, else
     // the register variant with 64-pixel tiles over 4 K-waves.
     const long long tiles32 = (g.m + 31) / 32;
-    // Up to 1024 tiles the automatic choice of the tile kernel needs no clock buffer set (it
-    // would have to hold this launch's stamps); the narrow kernel it stands in for does not.
-    const bool tile_pinned = ctx->fused_override.variant == dcn::kVariantTile || tiles32 > 1024;
-    const bool tile_ready = tile_pinned || !ctx->tile_clock;
     const bool bf16_window = packed->weights_group != nullptr && dcn::window_supported(*shape);
     const dcn::FusedConfig cfg =
         bf16 ? (tiles32 <= 1024 ? dcn::FusedConfig{dcn::kVariantNarrow, 1, 12, dcn::kSamplerBf16}
                 : bf16_window   ? dcn::FusedConfig{dcn::kVariantWindow, 4, 4, dcn::kSamplerBf16}
                                 : dcn::FusedConfig{dcn::kVariantRegister, 2, 4, dcn::kSamplerBf16})
              : choose_config(ctx->fused_override, g, *shape, packed->weights_group != nullptr && dcn::window_supported(*shape),
-                             tile_ready && packed->weights_tile != nullptr && dcn::tile_supported(*shape));
+                             packed->weights_tile != nullptr && dcn::tile_supported(*shape));
     if (!config_supported(cfg, g))
         return fail(ctx, DCN_INVALID_ARGUMENT,
                     "unsupported fused config (variant " + std::to_string(cfg.variant) + ", mt " +
                         std::to_string(cfg.mt) + ", ks " + std::to_string(cfg.ks) + ")");
     if (g.kb >= (1 << 16)) return fail(ctx, DCN_INVALID_SHAPE, "K too large for the fused path");
     const dcn::KShape ks = dcn::to_kshape(*shape);
-    if (cfg.variant == dcn::kVariantTile && ctx->tile_clock &&
-        ctx->tile_clock_count < 4 * dcn::tile_grid(ks, cfg))
+    // A clock buffer too small for this launch's stamps is an error, except up to 1024 tiles
+    // where the caller did not ask for the tile kernel: there the call goes on without stamps.
+    const bool clock_fits = cfg.variant == dcn::kVariantTile && ctx->tile_clock &&
+                            ctx->tile_clock_count >= 4 * dcn::tile_grid(ks, cfg);
+    const bool tile_asked = ctx->fused_override.variant == dcn::kVariantTile || tiles32 > 1024;
+    if (cfg.variant == dcn::kVariantTile && ctx->tile_clock && !clock_fits && tile_asked)
         return fail(ctx, DCN_INVALID_ARGUMENT,
                     "tile clock buffer holds " + std::to_string(ctx->tile_clock_count) +
                         " stamps; this launch needs " + std::to_string(4 * dcn::tile_grid(ks, cfg)));
@@ -211,7 +211,7 @@ dcn_status fused_prepacked_dev(dcn_context* ctx, const dcn_shape* shape, const v
             return fail(ctx, DCN_INVALID_ARGUMENT, "the tile variant does not support this shape");
         DCN_HIP(ctx, dcn::launch_tile_f16(ks, g, cfg, cb8, (const uint16_t*)d_offset,
                                           (const uint16_t*)d_mask, packed->weights_tile,
-                                          packed->bias, (uint16_t*)d_output, stream, ctx->tile_clock));
+                                          packed->bias, (uint16_t*)d_output, stream, clock_fits ? ctx->tile_clock : nullptr));
         return DCN_OK;
     }
     if (cfg.variant == dcn::kVariantNarrow) {

@@ -97,3 +97,25 @@ def test_pinned_narrow_settings_keep_the_narrow_kernel(gpu_ctx, dcn, torch, mt, 
         assert np.array_equal(outs[0], outs[1])
     finally:
         gpu_ctx.set_fused_config(0, 0, -1, 0)
+
+
+def test_clock_does_not_change_the_bits(gpu_ctx, dcn, torch):
+    """A clock buffer leaves choice and output as they are from 929 tiles on. Where the library
+    chose the tile kernel by itself, the call goes on without stamps if the buffer is too small for
+    them, up to 1024 tiles."""
+    print("case: tile clock", flush=True)
+    call = Call(torch, gpu_ctx, dcn, 8, 64, 64)
+    want, cfg = call.run(), gpu_ctx.get_fused_config(call.shape)
+    assert cfg["variant"] == TILE
+    need = 4 * 8 * 64 * 64 // 128  # four per 128-pixel tile
+    stamps = torch.zeros(need, dtype=torch.int64, device="cuda")
+    try:
+        for count in (need, need - 1, 1):
+            stamps.zero_()
+            gpu_ctx.set_tile_clock_dev(stamps, count)
+            assert gpu_ctx.get_fused_config(call.shape) == cfg
+            assert np.array_equal(call.run(), want)
+            started = stamps[0::4] != 0
+            assert bool(started.all()) if count == need else not bool(stamps.any())
+    finally:
+        gpu_ctx.set_tile_clock_dev(None)
