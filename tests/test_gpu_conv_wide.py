@@ -68,15 +68,15 @@ def test_wide_pair_same_bits(gpu_ctx, torch, h, w, acts, layouts, residuals):
     got = run(0)
     if CB8 in layouts[:residuals] + layouts[2:]:
         want = run(1)
-    else:  # no CB8 tensor to misalign: two single-conv calls
-        mid = _placed(torch, 8 * (h + 4) * (w + 4) * 8, 1)
-        out = _placed(torch, 64 * plane, 0)
+    else:  # no CB8 tensor to misalign: two single-conv calls with misaligned CB8 outputs
+        mid, out = (_placed(torch, 8 * (h + 4) * (w + 4) * 8, 1) for _ in range(2))
         r = [_dev(torch, a) for a in res]
         convs[0].run_dev(xd, mid, CB8, activation=acts[0])
         mid2 = mid.clone()
-        convs[1].run_dev(mid2, out, NCHW, activation=acts[1], res1=r[0], res1_layout=NCHW, res2=r[1], res2_layout=NCHW)
+        convs[1].run_dev(mid2, out, CB8, activation=acts[1], res1=r[0], res1_layout=NCHW, res2=r[1], res2_layout=NCHW)
         torch.cuda.synchronize()
-        want = out.cpu().numpy().view(np.uint16).copy()
+        blocks = out.cpu().numpy().view(np.uint16).reshape(8, h + 4, w + 4, 8)[:, 2:-2, 2:-2]
+        want = np.ascontiguousarray(blocks.transpose(0, 3, 1, 2)).ravel()
     for c in convs:
         c.free()
     a, b = got.view(np.float16), want.view(np.float16)
