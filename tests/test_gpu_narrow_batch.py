@@ -8,17 +8,6 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def dcn():
-    import jasnamacos_amd.deform_conv as module
-    return module
-
-
-@pytest.fixture(scope="module")
-def gpu_ctx(dcn):
-    return dcn.HipDeformConv(0)
-
-
 def case(dcn, batch, h, w):
     s = dcn.DeformConvShape(batch, 128, h, w, 64, h, w, 3, 3, 1, 1, 1, 1, 1, 1, 1, 16)
     rng = np.random.default_rng(batch * 1000 + h)
