@@ -365,8 +365,8 @@ __global__ __launch_bounds__(64 * (NW + SharedLayout<KA, CPI>::SW)) void shared_
 
     // Chain waves. This row's weights: chunk c of a stage is lane p's element 16 c + p of the
     // stage's (ic, tap) run. Channels past the group's load its last one. Elements past a
-    // channel's run, in the partial stage, are the next one's or, past the tensor, zero
-    // (the buffer's range check): nothing uses them.
+    // channel's run (in a partial stage) are the next one's or, past the tensor, zero (the
+    // buffer's range check): nothing uses them.
     const int oc0 = (blockIdx.y - group * a.oc_tiles) * (4 * NW * OCL) + (threadIdx.x >> 4) * OCL;  // in the group
     const __amdgpu_buffer_rsrc_t wr = dev::make_rsrc(a.weight, a.weight_bytes);
     uint32_t wbase[OCL];
@@ -388,9 +388,10 @@ __global__ __launch_bounds__(64 * (NW + SharedLayout<KA, CPI>::SW)) void shared_
         for (int e = 0; e < OCL; ++e) v[e] = load_widened<T>(wr, wbase[e] + (uint32_t)j0);
     };
     auto row4 = [&](int nb, int j) { return *reinterpret_cast<const float4*>(&sm[nb][p][j]); };
-    if (full > 0)
+    // The first stage unconditionally: under a branch the compiler converts FP16 weights as they
+    // are loaded, stage by stage (2x128x45x61 56.6 us against 47.9).
 #pragma unroll
-        for (int c = 0; c < KA; ++c) load_weights(0, c);
+    for (int c = 0; c < KA; ++c) load_run(16 * c, w[c]);
     __syncthreads();
 #pragma unroll 1
     for (int st = 0; st < full; ++st) {
