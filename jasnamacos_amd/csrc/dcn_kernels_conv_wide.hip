@@ -179,9 +179,10 @@ struct WidePair {
 // half of the output channels: a pixel fragment (LDS) serves two products and a weight
 // fragment (L1) up to P1. At 180 x 320 (240 tiles of 16 x 16, one per CU) 78 -> 17.3 us, 490
 // TFLOP/s, against conv_pair_kernel, whose 3,600 workgroups fetch all 148 KB of weights for 16
-// pixels each; 16 maps of 64 x 64 53 -> 22 us. What bounds it now: the LDS reads of the pixel
-// fragments (half a KB per product, as long as the product takes) and the latency of the two
-// dependent convs in one round of workgroups.
+// pixels each; 16 maps of 64 x 64 53 -> 18 us. No pipe is full (counters, per CU of 35.7 K cycles
+// at 180 x 320: matrix cores 32 %, other VALU 36 %, LDS 33 % with 45 % of that in bank conflicts,
+// addresser 48 %): with two waves per SIMD and one round of workgroups the time is the latency
+// of the copy and of two dependent convs.
 template <int TH, int PG>
 __global__ __launch_bounds__((64 * WidePair<TH, PG>::NW)) void conv_pair_wide_kernel(WidePairArgs a) {
     using L = WidePair<TH, PG>;
@@ -327,9 +328,10 @@ hipError_t launch_pair_wide(WidePairArgs a, int images, hipStream_t stream) {
 // every PG-th row by N of the NH * N 16-channel blocks.
 //
 // 3x3 over 16 maps of 64x64: 320 -> 64 channels 80.5 -> 31.8 us (760 TFLOP/s), 196 -> 64
-// 37.2 -> 19.1 us; 180x320 64 -> 432 130 -> 39.9 us. What bounds it: the weight fragments, 2 KB per
-// wave and K-step through the L1 for 4 or 8 products, and the pixel fragments, half a KB
-// of LDS per product with N = 2 (as long as the product takes), one with N = 1.
+// 37.2 -> 19.1 us; 180x320 64 -> 432 130 -> 39.9 us. What bounds it: the weight fragments through
+// the vector L1, 2 KB per wave and K-step for 4 or 8 products. The addresser is busy 88 % of the
+// time at 320 -> 64 (4 products) and 73 % at 196 -> 64 (8), the matrix cores 35 and
+// 41 %, the LDS 35 and 40 % (half of it bank conflicts).
 struct WideConvArgs {
     const void* xin;
     const void* wpk;
