@@ -475,12 +475,16 @@ dcn::KShape plainLayer(int cin, int h, int w, int cout, int kernel, int groups =
 }
 
 // A launch holds fewer than 2^32 threads along x. A 1x1 FP16 layer of three output channels
-// has 384 of them per 16 pixels on the shared-sample kernel: 178,956,970 pixels is the last
-// size that fits, and the tensors of the next ones are still within the library's limits.
+// has 384 of them per 16 output pixels on the shared-sample kernel: 178,956,960 pixels still fit,
+// and the tensors of the next sizes are within the library's limits. (32 input channels, so that
+// the choice by speed takes that kernel; its input may be smaller than its output.)
 TEST(cpu, sharedKernelGridStaysBelowTheThreadLimit) {
-    EXPECT(dcn::shared_forward_chosen(plainLayer(32, 1000, 1000, 3, 1), 2));
-    EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 8192, 21846, 3, 1), 2));  // 178,962,432
-    EXPECT(!dcn::shared_forward_chosen(plainLayer(1, 15000, 16000, 1, 1), 2));
+    dcn::KShape s = plainLayer(32, 64, 64, 3, 1);
+    s.Ho = 8192;
+    s.Wo = 21845;
+    EXPECT(dcn::shared_forward_chosen(s, 2));  // 178,954,240
+    s.Wo = 21846;
+    EXPECT(!dcn::shared_forward_chosen(s, 2));  // 178,962,432
 }
 
 // The shared-sample kernel's sampling positions are 32-bit integers, the other kernel's 64-bit:
