@@ -474,12 +474,12 @@ dcn::KShape plainLayer(int cin, int h, int w, int cout, int kernel, int groups =
     return {1, cin, h, w, cout, h, w, kernel, kernel, pad, pad, 1, 1, 1, 1, groups, offsetGroups};
 }
 
-// A launch holds fewer than 2^32 threads along x. A 1x1 FP16 layer of three output channels
+// A launch holds fewer than 2^32 threads along x. A 1x1 FP16 layer of two output channels
 // has 384 of them per 16 output pixels on the shared-sample kernel: 178,956,960 pixels still fit,
 // and the tensors of the next sizes are within the library's limits. (32 input channels, so that
 // the choice by speed takes that kernel; its input may be smaller than its output.)
 TEST(cpu, sharedKernelGridStaysBelowTheThreadLimit) {
-    dcn::KShape s = plainLayer(32, 64, 64, 3, 1);
+    dcn::KShape s = plainLayer(32, 64, 64, 2, 1);
     s.Ho = 8192;
     s.Wo = 21845;
     EXPECT(dcn::shared_forward_chosen(s, 2));  // 178,954,240
