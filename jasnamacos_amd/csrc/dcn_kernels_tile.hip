@@ -299,37 +299,41 @@ __device__ __forceinline__ void tile_copy_offsets(const TileArgs& a, __amdgpu_bu
 
 // The same for offsets or masks off 16-byte alignment, which the DMA's 16-byte pieces need:
 // through registers, by loads of any alignment (chunks past a tensor's end are zero, as
-// the DMA's range check leaves them). Each stage waits for the loads before their LDS writes.
-// us aligned / not, narrow kernel in brackets: 8 x 64x64 42.5 / 51.8 (56.7 / 58.3), with 32 px
-// flows 59.9 / 67.0 (62.3 / 62.7), 16 x 64x64 57.6 / 66.8.
+// the DMA's range check leaves them). A stage's loads are requested before its barrier and
+// written to LDS behind it, before its windows are requested. us aligned / not, narrow kernel in
+// brackets: 8 x 64x64 42.5 / 46.5 (56.4 / 58.2), with 32 px flows 59.1 / 63.8 (62.2 / 62.8), 16 x 64x64
+// 57.4 / 62.2.
+constexpr int kTileOffIter = (kTileOffCh * (kTilePix / 8) + 64 * kTileWaves - 1) / (64 * kTileWaves);
+struct TileOffsets {
+    u32x4 q[kTileOffIter];
+};
 template <int TW>
-__device__ __forceinline__ void tile_load_offsets(const TileArgs& a, int b, int ty, int tx, int st, uint8_t* dst,
-                                                  int wave, int lane) {
-    constexpr int NW = kTileWaves;
+__device__ __forceinline__ void tile_load_offsets(const TileArgs& a, int b, int ty, int tx, int st, int wave, int lane,
+                                                  TileOffsets& v) {
     constexpr int TH = kTilePix / TW;
     constexpr int kRowChunks = TW / 8;
     constexpr int kChunks = kTileOffCh * (kTilePix / 8);
     constexpr int kOffChunks = 36 * (kTilePix / 8);
-    constexpr int kIter = (kChunks + 64 * NW - 1) / (64 * NW);
     const int rem = lane % 16;
     const int y = min(ty * TH + rem / kRowChunks, a.Ho - 1);
     const int x = tx * TW + (rem % kRowChunks) * 8;
-    u32x4 q[kIter];
 #pragma unroll
-    for (int k = 0; k < kIter; ++k) {
-        const int c = (wave + k * NW) * 64 + lane;  // chunk: channel c / 16
+    for (int k = 0; k < kTileOffIter; ++k) {
+        const int c = (wave + k * kTileWaves) * 64 + lane;  // chunk: channel c / 16
         const bool is_off = c < kOffChunks;
         const uint32_t ch = is_off ? (uint32_t)(b * 2 * a.G * 9 + 36 * st) + c / 16
                                    : (uint32_t)(b * a.G * 9 + 18 * st) + c / 16 - 36;
         const uint32_t at = (ch * (uint32_t)a.HWo + (uint32_t)(y * a.Wo + x)) * 2u;  // bytes
-        q[k] = u32x4{0u, 0u, 0u, 0u};
+        v.q[k] = u32x4{0u, 0u, 0u, 0u};
         if (c < kChunks && at + 16u <= (is_off ? a.off_bytes : a.msk_bytes))
-            __builtin_memcpy(&q[k], reinterpret_cast<const uint8_t*>(is_off ? a.off : a.msk) + at, 16);
+            __builtin_memcpy(&v.q[k], reinterpret_cast<const uint8_t*>(is_off ? a.off : a.msk) + at, 16);
     }
+}
+__device__ __forceinline__ void tile_store_offsets(const TileOffsets& v, uint8_t* dst, int wave, int lane) {
 #pragma unroll
-    for (int k = 0; k < kIter; ++k) {
-        const int c = (wave + k * NW) * 64 + lane;
-        if (c < kChunks) *reinterpret_cast<u32x4*>(dst + c * 16) = q[k];
+    for (int k = 0; k < kTileOffIter; ++k) {
+        const int c = (wave + k * kTileWaves) * 64 + lane;
+        if (c < kTileOffCh * (kTilePix / 8)) *reinterpret_cast<u32x4*>(dst + c * 16) = v.q[k];
     }
 }
 
@@ -535,10 +539,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void tile_kernel(TileArgs a) {
             ybf[s][t] = (float)(ybi[s] + t * a.dh);
             xbf[s][t] = (float)(xbi[s] + t * a.dw);
         }
-    auto copy_offsets = [&](int st) {
-        if constexpr (DMA) tile_copy_offsets<TW>(a, orr, mr, b, ty, tx, st, offs, wave, lane);
-        else tile_load_offsets<TW>(a, b, ty, tx, st, offs, wave, lane);
-    };
+    auto copy_offsets = [&](int st) { tile_copy_offsets<TW>(a, orr, mr, b, ty, tx, st, offs, wave, lane); };
 
     // Window geometry of a stage (wave-uniform): origin, size in units, LDS placement.
     struct Win {
@@ -810,11 +811,17 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void tile_kernel(TileArgs a) {
         Win win;
         Addressing ad;
         auto next_stage = [&](int st1, Samples& C) {
+            TileOffsets next;
+            if constexpr (!DMA)
+                if (st1 + 1 < stages) tile_load_offsets<TW>(a, b, ty, tx, st1 + 1, wave, lane, next);
             publish_box();
             __syncthreads();  // every box; every wave past its corner and offset reads
             win = read_windows();
+            if constexpr (!DMA)
+                if (st1 + 1 < stages) tile_store_offsets(next, offs, wave, lane);
             copy_windows(st1, win, win.split ? 0 : -1);
-            if (st1 + 1 < stages) copy_offsets(st1 + 1);
+            if constexpr (DMA)
+                if (st1 + 1 < stages) copy_offsets(st1 + 1);
             ad = addressing(st1, win);
 #pragma unroll
             for (int j = 0; j < NSMP; ++j) make_address(j, C, ad);
@@ -836,7 +843,13 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void tile_kernel(TileArgs a) {
                 load_b(0, slot);
             }
         }
-        if (!pair_plan) copy_offsets(0);
+        if constexpr (!DMA) {
+            TileOffsets first;
+            tile_load_offsets<TW>(a, b, ty, tx, 0, wave, lane, first);
+            tile_store_offsets(first, offs, wave, lane);
+        } else if (!pair_plan) {
+            copy_offsets(0);
+        }
         if (tid < 8) reinterpret_cast<uint32_t*>(lds + kTileZero)[tid] = 0u;
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // stage 0's offsets in LDS; the zero bytes
